@@ -8,9 +8,10 @@
  *     (1..NC), NK = ceil(NC / G).  K, F and FF are multiples of 16 with
  *     K <= 64, F <= 256, FF <= 1024.  K = 16 with F in {32, 64} (and, for the
  *     MLP, FF in {64, 128, 256}) runs the specialised kernels; every other
- *     shape runs the general-shape kernels, whose forward also needs the
- *     `saved` buffer (it holds the state entering every mini-batch and the
- *     per-mini-batch scratch; the backward reads it).  The fixed-weight
+ *     shape runs the general-shape kernels or those for a subset of their
+ *     shapes, whose forward also needs the `saved` buffer (it holds the state
+ *     entering every mini-batch and the per-mini-batch scratch; the backward
+ *     reads and writes it).  The fixed-weight
  *     kernels (cached readout, memo combiner) take any K, F in {32, 64} and
  *     FF in {32, 64, 128, 256}.
  *   - Activations (XQ, XK, XV, out and their gradients) share one dtype,
@@ -99,7 +100,10 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
 /* Bytes of the saved buffer of ttt_linear_fwd / ttt_linear_bwd: with the
  * specialised kernels B*H*NC mini-batches x (3 * F * 64 + 256); with the
  * general-shape kernels, per chain, the state entering every mini-batch and
- * the fp32 scratch of one mini-batch; 0 for unsupported sizes. */
+ * the fp32 scratch of one mini-batch; with K in {32, 48, 64} and F = 64, per
+ * mini-batch, the state entering it (F F + F), 4 K F of forward values and of
+ * the backward's handoff, F F + 3 F + 2 K more of the handoff, all fp32; 0 for
+ * unsupported sizes. */
 size_t ttt_linear_saved_bytes(int B, int H, int NC, int K, int F);
 
 /* TTT-Linear backward: gradients of sum(out * dout) wrt every input, the
@@ -156,7 +160,9 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
  * specialised kernels B*H*NC mini-batches x ((7 FF + F) * K * sizeof(dtype)
  * + (FF + F) * 4 + 3 * F * 64 + 4096); with the general-shape kernels, per
  * chain, the state entering every mini-batch and the fp32 scratch of one
- * mini-batch. */
+ * mini-batch; with K in {32, 48, 64} and (F, FF) one of (64, 64), (64, 256)
+ * and (32, 128), per mini-batch, twice the state (2 F FF + FF + F), 4 K (FF + F)
+ * of forward values and of the backward's handoff, and 2 F + 2 K, all fp32. */
 size_t ttt_mlp_saved_bytes(int B, int H, int NC, int K, int F, int FF, int dtype);
 
 /* Bytes of device workspace ttt_mlp_bwd uses: B*H*NC mini-batches x

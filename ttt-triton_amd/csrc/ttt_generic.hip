@@ -4,7 +4,9 @@
 // (those hold K = 16 and F in {32, 64} in registers, FF in {64, 128, 256}).
 // This is what the reference's own model configuration needs: TTTMLP sets
 // FF = F (ttt_layer.py:427-430) and ModelConfig defaults to K = 64 with
-// F = 32 (forecast.py:33-44).
+// F = 32 (forecast.py:33-44).  Of the general-shape set, F = FF = 32 runs the
+// register-resident kernels (ttt_small.hip) and mini-batches of 32 to 64
+// tokens on 64-wide heads the kernels of ttt_wide.h; the rest runs these.
 //
 // One workgroup of 256 threads per (batch, head) chain walks the mini-batches
 // in order (ops/ttt_linear.py:8-54, ops/ttt_mlp.py:9-67, dual form with the
@@ -826,11 +828,13 @@ bool gen_shape_ok(int K, int F, int FF, bool mlp) {
 }
 
 size_t gen_saved_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp) {
+  if (wide_shape_ok(K, F, FF, mlp)) return wide_saved_bytes(B, H, NC, K, F, FF, mlp);
   return (size_t)B * H * GenLayout(K, F, FF, NC, mlp).per_chain * sizeof(float);
 }
 
 hipError_t launch_gen_fwd(const GenFwdParams& q, int dtype, hipStream_t stream) {
   if (small_shape_ok(q.K, q.F, q.FF, q.mlp) && !gen_force_general()) return launch_small_fwd(q, dtype, stream);
+  if (wide_shape_ok(q.K, q.F, q.FF, q.mlp)) return launch_wide_fwd(q, dtype, stream);
   GenArgs a{};
   a.XQ = q.XQ;
   a.XK = q.XK;
@@ -865,6 +869,7 @@ hipError_t launch_gen_fwd(const GenFwdParams& q, int dtype, hipStream_t stream) 
 
 hipError_t launch_gen_bwd(const GenBwdParams& q, int dtype, hipStream_t stream) {
   if (small_shape_ok(q.K, q.F, q.FF, q.mlp) && !gen_force_general()) return launch_small_bwd(q, dtype, stream);
+  if (wide_shape_ok(q.K, q.F, q.FF, q.mlp)) return launch_wide_bwd(q, dtype, stream);
   GenArgs a{};
   a.XQ = q.XQ;
   a.XK = q.XK;

@@ -255,6 +255,12 @@ bool small_shape_ok(int K, int F, int FF, bool mlp);
 // workspace bytes of the register-resident MLP backward's two-launch form
 // (0 for K outside 16..64); a smaller workspace runs the one-launch form
 size_t small_mlp_bwd_hand_bytes(int B, int H, int NC, int K);
+// mini-batch-in-LDS kernels (ttt_wide.h) for K = 32, 48, 64 with F = 64 (MLP:
+// FF = 64 or 256, or F = 32 with FF = 128), their own slots in `saved`
+bool wide_shape_ok(int K, int F, int FF, bool mlp);
+size_t wide_saved_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp);
+hipError_t launch_wide_fwd(const GenFwdParams& p, int dtype, hipStream_t stream);
+hipError_t launch_wide_bwd(const GenBwdParams& p, int dtype, hipStream_t stream);
 bool gen_force_general();  // TTT_OPT_SMALL_KERNELS = 0: always the staged general-shape kernels
 hipError_t launch_small_fwd(const GenFwdParams& p, int dtype, hipStream_t stream);
 hipError_t launch_small_bwd(const GenBwdParams& p, int dtype, hipStream_t stream);

@@ -1,0 +1,216 @@
+// TTT inner loops of mini-batches of 32, 48 or 64 tokens on 64-wide heads (and
+// of the 32-wide MLP with 128 hidden units): one workgroup holds a whole
+// mini-batch in LDS and every product is 16 x 16 output tiles of fp32 MFMA,
+// one K x 64 tile per wave.
+//
+// What bounds the shape is the recurrence: B*H chains, each NC mini-batches in
+// a row, so a launch has B*H workgroups however long the sequence.  Only the
+// products that the next mini-batch's state needs are therefore left in the
+// per-chain launch; the readout, which reads a state and writes nothing that
+// a later mini-batch reads, runs as a second launch with one workgroup per
+// (chain, mini-batch), forward and backward alike:
+//   wide_fwd_state    per chain: Z1, X2, Z2, G2, P = G2 W2^T, the update
+//   wide_fwd_readout  per (chain, mini-batch): A1, Z1b, A2, Z2b, the output
+//   wide_bwd_readout  per (chain, mini-batch): the readout again and its
+//                     gradients: dXQ, most of deta, and what it adds to dG1,
+//                     dG2, dX2, dXK, dW and db (the handoff)
+//   wide_bwd_state    per chain, mini-batches in reverse: the update's gradient
+// (the Linear loop has one layer: G, no P; the same four launches.)
+//
+// Measured at B32 H4, 8 mini-batches of 64 tokens, F = FF = 64, bf16, forward +
+// backward: 511 us (MLP; state 78 + 247, readouts 54 + 132), where the
+// general-shape kernels (one workgroup per chain for everything, every matrix
+// through global scratch) take 6,780; the Linear loop 201 us against 3,090.
+// The shapes taken are those that a layer (FF = F) or the 4x MLP builds of
+// 32- and 64-wide heads; others keep the general-shape kernels.
+//
+// Everything is held and summed in fp32 whatever the activation type, as in
+// the general-shape kernels (ttt_generic.hip); activations are converted on
+// load.  `saved` holds one slot per (chain, mini-batch), WideSlot below.
+#pragma once
+
+#include "ttt_eta.h"
+#include "ttt_kernels.h"
+
+namespace ttt {
+
+// K = 16 KT tokens, F = 16 FT features, hidden units in NSL slices of 64
+// (the Linear loop: one "slice", its F = 64 output columns).
+template <int KT_, int FT_, int NSL_, bool MLP_> struct WideShape {
+  static constexpr int KT = KT_, FT = FT_, NSL = NSL_;
+  static constexpr bool MLP = MLP_;
+  static constexpr int K = 16 * KT, F = 16 * FT, S = 64, FF = S * NSL;
+  static constexpr int NW = 4 * KT;        // waves: the 16 x 16 tiles of a K x 64 product
+  static constexpr int NTH = 64 * NW;      // 16 threads per token row
+  static constexpr int V = F / 16;         // features per thread in a row pass
+  static constexpr int TW = FT * 4;        // 16 x 16 tiles of one slice of W1 or W2
+  static constexpr int NT = (TW + NW - 1) / NW;  // of those, per wave
+  // LDS rows are padded by 4 floats: row-major float4 reads (16 rows x 4 lane
+  // groups) and column reads (4 rows x 16 lanes) both touch 64 distinct banks
+  static constexpr int LS = S + 4, LF = F + 4, LK = K + 4;
+  static constexpr int SLOT = 64 * LS;     // one LDS matrix of up to 64 x 64
+  static_assert(MLP || (FT == 4 && NSL == 1), "the Linear loop: 64 features, one slice");
+};
+
+// floats of one (chain, mini-batch) slot of `saved`
+template <class C> struct WideSlot {
+  static constexpr int STATE = C::MLP ? 2 * C::F * C::FF + C::FF + C::F : C::F * C::F + C::F;
+  // the state entering the mini-batch
+  static constexpr int W1 = 0;
+  static constexpr int B1 = C::MLP ? C::F * C::FF : C::F * C::F;
+  static constexpr int W2 = B1 + (C::MLP ? C::FF : C::F);
+  static constexpr int B2 = W2 + C::FF * C::F;
+  // written by wide_fwd_state: Z1 + b1 and P = G2 W2^T (MLP), G2 (Linear: G),
+  // the normalised Z2 (Linear: Z) and its sigma
+  static constexpr int Z1 = STATE;
+  static constexpr int P = Z1 + (C::MLP ? C::K * C::FF : 0);
+  static constexpr int G2 = P + (C::MLP ? C::K * C::FF : 0);
+  static constexpr int ZH = G2 + C::K * C::F;
+  static constexpr int SIG = ZH + C::K * C::F;
+  // the handoff from wide_bwd_readout to wide_bwd_state: the readout's terms
+  // of dG1, dX2, dG2, dXK, the state gradient, the LayerNorm parameters'
+  // gradients, and deta's last row (for an lr rule: dlr)
+  static constexpr int HG1 = SIG + C::K;
+  static constexpr int HX2 = HG1 + (C::MLP ? C::K * C::FF : 0);
+  static constexpr int HG2 = HX2 + (C::MLP ? C::K * C::FF : 0);
+  static constexpr int HXK = HG2 + C::K * C::F;
+  static constexpr int HST = HXK + C::K * C::F;  // dW1, db1[, dW2, db2] laid out as the state
+  static constexpr int HLW = HST + STATE;
+  static constexpr int HLB = HLW + C::F;
+  static constexpr int HDE = HLB + C::F;
+  static constexpr int FLOATS = HDE + C::K;
+};
+
+struct WideArgs {
+  const void *XQ, *XK, *XV, *eta, *dout;
+  const float *ln_w, *ln_b;
+  const float *W1_init, *b1_init, *W2_init, *b2_init;
+  void* out;
+  float *W1_last, *b1_last, *W2_last, *b2_last;
+  float *W1_ckpt, *b1_ckpt, *W2_ckpt, *b2_ckpt;
+  float *W1_memo, *b1_memo, *W2_memo, *b2_memo;
+  void *dXQ, *dXK, *dXV, *deta;
+  float *dW1, *db1, *dW2, *db2, *dln_w, *dln_b;
+  float* saved;
+  int H, NC, G, M, eta_rule;
+  float eps;
+};
+
+// ---------------------------------------------------------------- products
+// c + op(A) op(B) for one 16 x 16 output tile, contraction KD (a multiple of
+// 16): A and B point at the tile's first row (column) of op(A) (op(B)) in
+// LDS.  op(A)[i][k] = TA ? A[k * LA + i] : A[i * LA + k], op(B)[k][j] = TB ?
+// B[j * LB + k] : B[k * LB + j].  fp32 MFMA with the operands swapped, so that
+// lane (g, r) holds C[r][4g .. 4g + 3]: four consecutive columns of one row
+// (16-byte LDS and global accesses, per-row factors one scalar per lane).
+// With CS, `cs` receives op(B)'s column sums (column r, in every lane group).
+template <int KD, bool TA, bool TB, int LA, int LB, bool CS = false>
+__device__ __forceinline__ f4 wmm(f4 c, const float* A, const float* B, float* cs = nullptr) {
+  const int l = lane_id(), g = l >> 4, r = l & 15;
+  const float* ap = TA ? A + 4 * g * LA + r : A + r * LA + 4 * g;
+  const float* bp = TB ? B + r * LB + 4 * g : B + 4 * g * LB + r;
+  float t = 0.f;
+#pragma unroll
+  for (int k = 0; k < KD; k += 16) {
+    Frag<float> a, b;
+    if constexpr (TA) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a.v[j] = ap[(k + j) * LA];
+    } else {
+      a.v = *reinterpret_cast<const f4*>(ap + k);
+    }
+    if constexpr (TB) {
+      b.v = *reinterpret_cast<const f4*>(bp + k);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b.v[j] = bp[(k + j) * LB];
+    }
+    if constexpr (CS) t += (b.v[0] + b.v[1]) + (b.v[2] + b.v[3]);
+    mma16(c, b, a);
+  }
+  if constexpr (CS) *cs = sum_col4(t);
+  return c;
+}
+
+// the 16 x 16 tile grid of an R x Cc-tile product over the waves: tile w
+template <int CT> struct WideTile {
+  int it, jt;
+  __device__ __forceinline__ explicit WideTile(int t) : it(t / CT), jt(t % CT) {}
+  __device__ __forceinline__ int row() const { return 16 * it + (lane_id() & 15); }
+  __device__ __forceinline__ int col() const { return 16 * jt + 4 * (lane_id() >> 4); }
+};
+
+// ---------------------------------------------------------------- loads, stores
+__device__ __forceinline__ f4 ldf4(const float* p) { return *reinterpret_cast<const f4*>(p); }
+__device__ __forceinline__ void stf4(float* p, f4 v) { *reinterpret_cast<f4*>(p) = v; }
+
+template <typename T> __device__ __forceinline__ Frag<T> ldraw4(const T* p) {
+  Frag<T> f;
+  f.v = *reinterpret_cast<const typename FragT<T>::type*>(p);
+  return f;
+}
+template <typename T> __device__ __forceinline__ void st4(T* p, f4 v) {
+  *reinterpret_cast<typename FragT<T>::type*>(p) = to_frag<T>(v).v;
+}
+
+// V = 2 or 4 consecutive values of a row pass
+template <int V> struct VecF { typedef float type __attribute__((ext_vector_type(V))); };
+template <typename T, int V> struct VecT { typedef T type __attribute__((ext_vector_type(V))); };
+template <int V> __device__ __forceinline__ typename VecF<V>::type ldv(const float* p) {
+  return *reinterpret_cast<const typename VecF<V>::type*>(p);
+}
+template <int V> __device__ __forceinline__ void stv(float* p, typename VecF<V>::type v) {
+  *reinterpret_cast<typename VecF<V>::type*>(p) = v;
+}
+template <typename T, int V> __device__ __forceinline__ typename VecT<T, V>::type ldact(const T* p) {
+  return *reinterpret_cast<const typename VecT<T, V>::type*>(p);
+}
+template <typename T, int V> __device__ __forceinline__ typename VecF<V>::type actf(typename VecT<T, V>::type x) {
+  typename VecF<V>::type y;
+#pragma unroll
+  for (int q = 0; q < V; ++q) y[q] = (float)x[q];
+  return y;
+}
+template <typename T, int V> __device__ __forceinline__ void stact(T* p, typename VecF<V>::type v) {
+  f4 x = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < V; ++q) x[q] = v[q];
+  const Frag<T> f = to_frag<T>(x);
+  typename VecT<T, V>::type y;
+#pragma unroll
+  for (int q = 0; q < V; ++q) y[q] = f.v[q];
+  *reinterpret_cast<typename VecT<T, V>::type*>(p) = y;
+}
+
+// eta[K - 1][j] of a mini-batch whose eta (lr) starts at row0 = slot * K
+template <typename T, int K> __device__ __forceinline__ float wide_eta_last(const WideArgs& a, size_t slot, int j) {
+  if (a.eta_rule == TTT_ETA_DENSE) return (float)static_cast<const T*>(a.eta)[(slot * K + (K - 1)) * K + j];
+  const float* e = static_cast<const float*>(a.eta);
+  if (a.eta_rule == TTT_ETA_DENSE_F32) return e[(slot * K + (K - 1)) * K + j];
+  return e[slot * K + j] * (1.0f / (float)K);
+}
+// eta[i][j .. j + 3]
+template <typename T, int K> __device__ __forceinline__ f4 wide_eta4(const WideArgs& a, size_t slot, int i, int j) {
+  if (a.eta_rule == TTT_ETA_DENSE) return frag_to_f4(ldraw4(static_cast<const T*>(a.eta) + (slot * K + i) * K + j));
+  const float* e = static_cast<const float*>(a.eta);
+  if (a.eta_rule == TTT_ETA_DENSE_F32) return ldf4(e + (slot * K + i) * K + j);
+  const f4 lr = ldf4(e + slot * K + j);
+  if (a.eta_rule == TTT_ETA_LAYER) return lr * (1.0f / (float)K);
+  const float c = 1.0f / (float)(i + 1);
+  f4 r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = j + q <= i ? lr[q] * c : 0.f;
+  return r;
+}
+// coefficient of lr[j] in eta[i][j]
+template <int K> __device__ __forceinline__ float wide_eta_coef(int rule, int i, int j) {
+  if (rule == TTT_ETA_LAYER) return 1.0f / (float)K;
+  return j <= i ? 1.0f / (float)(i + 1) : 0.f;
+}
+
+// ---------------------------------------------------------------- launchers
+// one translation unit per activation type (ttt_wide_{f32,bf16,f16}.hip)
+template <typename T>
+hipError_t launch_wide_t(const WideArgs& a, int K, int F, int FF, bool mlp, bool bwd, int chains, hipStream_t stream);
+
+}  // namespace ttt
