@@ -258,7 +258,8 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
     const vf zh = ldv<V>(slot + Sl::ZH + prow * F + pcol);
     const float sd = slot[Sl::SIG + prow];
     const float e_s = wide_eta_last<T, K>(a, m, ts.row());
-    const float e_f = C::FT == 4 ? e_s : wide_eta_last<T, K>(a, m, tf.row());
+    // (waves without a K x F tile have rows past the mini-batch, and past eta's end at the last one)
+    const float e_f = C::FT == 4 ? e_s : has_f ? wide_eta_last<T, K>(a, m, tf.row()) : 0.f;
     if (tid < 2 * F) hln += slot[Sl::HLW + tid];  // (HLB follows HLW)
     const vf xk = actf<T, V>(rxk), g2 = rg2;
     stv<V>(XKs + prow * LF + pcol, xk);
