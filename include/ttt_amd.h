@@ -55,6 +55,14 @@ enum ttt_dtype { TTT_DTYPE_F32 = 0, TTT_DTYPE_BF16 = 1, TTT_DTYPE_F16 = 2 };
 
 enum ttt_eta_rule { TTT_ETA_DENSE = 0, TTT_ETA_LAYER = 1, TTT_ETA_CAUSAL = 2, TTT_ETA_DENSE_F32 = 3 };
 
+/* May be or'ed into the eta_rule of ttt_linear_fwd / _bwd and ttt_mlp_fwd / _bwd
+ * with TTT_DTYPE_F32 where ttt_split_saved_bytes is not 0: the split form,
+ * whose per-chain launch carries the state alone and whose readout (and its
+ * gradients) is a second launch with a workgroup per (chain, mini-batch).
+ * Faster where few chains leave the GPU idle.  It takes a `saved` buffer of ttt_split_saved_bytes in every call (the backward reads and writes
+ * the forward's), no checkpoints, final state or workspace in the backward. */
+enum ttt_form { TTT_FORM_SPLIT = 0x100 };
+
 enum ttt_status {
   TTT_OK = 0,
   TTT_ERR_SHAPE = -1,     /* unsupported or inconsistent shape */
@@ -105,6 +113,10 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
  * the backward's handoff, F F + 3 F + 2 K more of the handoff, all fp32; 0 for
  * unsupported sizes. */
 size_t ttt_linear_saved_bytes(int B, int H, int NC, int K, int F);
+
+/* Bytes of the saved buffer of the split form (TTT_FORM_SPLIT; FF = 0: the
+ * Linear loop): K = 16 with F = 64 (MLP: FF = 64, or F = 32 with FF = 128); 0 for any other shape. */
+size_t ttt_split_saved_bytes(int B, int H, int NC, int K, int F, int FF);
 
 /* TTT-Linear backward: gradients of sum(out * dout) wrt every input, the
  * final state's gradient taken as zero (the ops path discards W_last).

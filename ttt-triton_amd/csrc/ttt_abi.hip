@@ -23,6 +23,12 @@ std::atomic<long long> g_small_kernels{1};
 bool eta_rule_ok(int r) {
   return r == TTT_ETA_DENSE || r == TTT_ETA_LAYER || r == TTT_ETA_CAUSAL || r == TTT_ETA_DENSE_F32;
 }
+// TTT_FORM_SPLIT, taken off the eta rule that carries it
+bool take_split(int& eta_rule) {
+  const bool split = (eta_rule & TTT_FORM_SPLIT) != 0;
+  eta_rule &= ~TTT_FORM_SPLIT;
+  return split;
+}
 // fp32 dense eta under fp32 activations is the plain dense form
 int eta_rule_of(int r, int dtype) { return r == TTT_ETA_DENSE_F32 && dtype == TTT_DTYPE_F32 ? TTT_ETA_DENSE : r; }
 
@@ -140,10 +146,15 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
                    float* W1_ckpt, float* b1_ckpt, void* saved, size_t saved_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
+  const bool split = take_split(eta_rule);
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
   eta_rule = eta_rule_of(eta_rule, dtype);
-  st = fast_linear_shape(K, F) ? check_linear(NC, F) : TTT_OK;
+  const bool fast = fast_linear_shape(K, F) && !split;
+  st = fast ? check_linear(NC, F) : TTT_OK;
   if (st != TTT_OK) return st;
+  const size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, 0) : ttt_linear_saved_bytes(B, H, NC, K, F);
+  if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
+  if (split && need == 0) return TTT_ERR_SHAPE;
   REQUIRE_PTR(XQ);
   REQUIRE_PTR(XK);
   REQUIRE_PTR(XV);
@@ -161,9 +172,9 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
   if ((W1_ckpt == nullptr) != (b1_ckpt == nullptr)) return TTT_ERR_NULL;
   if (saved != nullptr) {
     if (!aligned16(saved)) return TTT_ERR_ALIGN;
-    if (saved_bytes < ttt_linear_saved_bytes(B, H, NC, K, F)) return TTT_ERR_WORKSPACE;
+    if (saved_bytes < need) return TTT_ERR_WORKSPACE;
   }
-  if (!fast_linear_shape(K, F)) {
+  if (!fast) {
     if (saved == nullptr) return TTT_ERR_WORKSPACE;  // the general path's states and scratch
     ttt::GenFwdParams q{};
     q.XQ = XQ;
@@ -191,7 +202,8 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
     q.eta_rule = eta_rule;
     q.mlp = false;
     q.eps = eps;
-    return hip_status(ttt::launch_gen_fwd(q, dtype, static_cast<hipStream_t>(stream)));
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    return hip_status(split ? ttt::launch_wide_fwd(q, dtype, hs) : ttt::launch_gen_fwd(q, dtype, hs));
   }
 
   ttt::LinearFwdParams p;
@@ -227,18 +239,25 @@ int ttt_linear_bwd(const void* XQ, const void* XK, const void* XV, const void* e
                    size_t saved_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
+  const bool split = take_split(eta_rule);
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
   eta_rule = eta_rule_of(eta_rule, dtype);
-  st = fast_linear_shape(K, F) ? check_linear(NC, F) : TTT_OK;
+  const bool fast = fast_linear_shape(K, F) && !split;
+  st = fast ? check_linear(NC, F) : TTT_OK;
   if (st != TTT_OK) return st;
+  const size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, 0) : ttt_linear_saved_bytes(B, H, NC, K, F);
+  if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
+  if (split && need == 0) return TTT_ERR_SHAPE;
   REQUIRE_PTR(XQ);
   REQUIRE_PTR(XK);
   REQUIRE_PTR(XV);
   REQUIRE_PTR(eta);
   REQUIRE_PTR(ln_w);
   REQUIRE_PTR(ln_b);
-  REQUIRE_PTR(W1_ckpt);
-  REQUIRE_PTR(W1_last);
+  if (!split) {  // (the split form's slots hold every mini-batch's state)
+    REQUIRE_PTR(W1_ckpt);
+    REQUIRE_PTR(W1_last);
+  }
   REQUIRE_PTR(dout);
   REQUIRE_PTR(dXQ);
   REQUIRE_PTR(dXK);
@@ -250,8 +269,8 @@ int ttt_linear_bwd(const void* XQ, const void* XK, const void* XV, const void* e
   REQUIRE_PTR(dln_b);
   if (saved == nullptr) return TTT_ERR_WORKSPACE;
   if (!aligned16(saved)) return TTT_ERR_ALIGN;
-  if (saved_bytes < ttt_linear_saved_bytes(B, H, NC, K, F)) return TTT_ERR_WORKSPACE;
-  if (!fast_linear_shape(K, F)) {
+  if (saved_bytes < need) return TTT_ERR_WORKSPACE;
+  if (!fast) {
     ttt::GenBwdParams q{};
     q.XQ = XQ;
     q.XK = XK;
@@ -278,7 +297,8 @@ int ttt_linear_bwd(const void* XQ, const void* XK, const void* XV, const void* e
     q.eta_rule = eta_rule;
     q.mlp = false;
     q.eps = eps;
-    return hip_status(ttt::launch_gen_bwd(q, dtype, static_cast<hipStream_t>(stream)));
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    return hip_status(split ? ttt::launch_wide_bwd(q, dtype, hs) : ttt::launch_gen_bwd(q, dtype, hs));
   }
 
   ttt::LinearBwdParams p;
@@ -318,8 +338,13 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
                 float* b2_memo, void* saved, size_t saved_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
-  const bool fast = fast_mlp_shape(K, F, FF);
+  const bool split = take_split(eta_rule);
+  const bool fast = fast_mlp_shape(K, F, FF) && !split;
   if (!fast && !ttt::gen_shape_ok(K, F, FF, true)) return TTT_ERR_SHAPE;
+  const size_t need =
+      split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) : ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype);
+  if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
+  if (split && need == 0) return TTT_ERR_SHAPE;
   st = fast ? check_mlp(NC, F, FF, dtype) : TTT_OK;
   if (st != TTT_OK) return st;
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
@@ -348,7 +373,7 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
   if (W1_memo != nullptr && M < 1) return TTT_ERR_ARG;
   if (saved != nullptr) {
     if (!aligned16(saved)) return TTT_ERR_ALIGN;
-    if (saved_bytes < ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype)) return TTT_ERR_WORKSPACE;
+    if (saved_bytes < need) return TTT_ERR_WORKSPACE;
   }
   if (!fast) {
     if (saved == nullptr) return TTT_ERR_WORKSPACE;  // the general path's states and scratch
@@ -388,7 +413,8 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
     q.eta_rule = eta_rule;
     q.mlp = true;
     q.eps = eps;
-    return hip_status(ttt::launch_gen_fwd(q, dtype, static_cast<hipStream_t>(stream)));
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    return hip_status(split ? ttt::launch_wide_fwd(q, dtype, hs) : ttt::launch_gen_fwd(q, dtype, hs));
   }
 
   ttt::MlpFwdParams p;
@@ -428,6 +454,11 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
   p.eta_rule = eta_rule;
   p.eps = eps;
   return hip_status(ttt::launch_mlp_fwd(p, dtype, static_cast<hipStream_t>(stream)));
+}
+
+size_t ttt_split_saved_bytes(int B, int H, int NC, int K, int F, int FF) {
+  if (B <= 0 || H <= 0 || NC <= 0 || K != 16) return 0;
+  return ttt::wide_saved_bytes(B, H, NC, K, F, FF > 0 ? FF : F, FF > 0);
 }
 
 size_t ttt_mlp_saved_bytes(int B, int H, int NC, int K, int F, int FF, int dtype) {
@@ -470,8 +501,13 @@ static int mlp_bwd_impl(const void* XQ, const void* XK, const void* XV, const vo
                 size_t workspace_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
-  const bool fast = fast_mlp_shape(K, F, FF);
+  const bool split = take_split(eta_rule);
+  const bool fast = fast_mlp_shape(K, F, FF) && !split;
   if (!fast && !ttt::gen_shape_ok(K, F, FF, true)) return TTT_ERR_SHAPE;
+  const size_t need =
+      split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) : ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype);
+  if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
+  if (split && need == 0) return TTT_ERR_SHAPE;
   st = fast ? check_mlp(NC, F, FF, dtype) : TTT_OK;
   if (st != TTT_OK) return st;
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
@@ -479,16 +515,20 @@ static int mlp_bwd_impl(const void* XQ, const void* XK, const void* XV, const vo
   (void)b1_ckpt;  // not read: the saved values carry the rest of the state
   (void)W2_ckpt;
   (void)b2_ckpt;
-  const void* req[] = {XQ, XK, XV, eta, ln_w, ln_b, W1_ckpt,
-                       W1_last, b1_last, W2_last, b2_last, dout,
-                       dXQ, dXK, dXV, deta, dW1, db1, dW2, db2, dln_w, dln_b};
+  const void* req[] = {XQ, XK, XV, eta, ln_w, ln_b, dout, dXQ, dXK, dXV, deta, dW1, db1, dW2, db2, dln_w, dln_b};
   for (const void* q : req) REQUIRE_PTR(q);
+  if (!split)  // (the split form's slots hold every mini-batch's state)
+    for (const void* q : {(const void*)W1_ckpt, (const void*)W1_last, (const void*)b1_last, (const void*)W2_last,
+                          (const void*)b2_last})
+      REQUIRE_PTR(q);
   if (saved == nullptr) return TTT_ERR_WORKSPACE;
   if (!aligned16(saved)) return TTT_ERR_ALIGN;
-  if (saved_bytes < ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype)) return TTT_ERR_WORKSPACE;
-  if (workspace == nullptr) return TTT_ERR_WORKSPACE;
-  if (!aligned16(workspace)) return TTT_ERR_ALIGN;
-  if (workspace_bytes < mlp_bwd_min_workspace(B, H, NC, K, F, FF, dtype)) return TTT_ERR_WORKSPACE;
+  if (saved_bytes < need) return TTT_ERR_WORKSPACE;
+  if (!split) {
+    if (workspace == nullptr) return TTT_ERR_WORKSPACE;
+    if (!aligned16(workspace)) return TTT_ERR_ALIGN;
+    if (workspace_bytes < mlp_bwd_min_workspace(B, H, NC, K, F, FF, dtype)) return TTT_ERR_WORKSPACE;
+  }
   if (!fast) {
     ttt::GenBwdParams q{};
     q.ws = workspace;
@@ -520,7 +560,8 @@ static int mlp_bwd_impl(const void* XQ, const void* XK, const void* XV, const vo
     q.eta_rule = eta_rule;
     q.mlp = true;
     q.eps = eps;
-    return hip_status(ttt::launch_gen_bwd(q, dtype, static_cast<hipStream_t>(stream)));
+    hipStream_t hs = static_cast<hipStream_t>(stream);
+    return hip_status(split ? ttt::launch_wide_bwd(q, dtype, hs) : ttt::launch_gen_bwd(q, dtype, hs));
   }
 
   ttt::MlpBwdParams p;

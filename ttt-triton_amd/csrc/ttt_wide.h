@@ -1,4 +1,4 @@
-// TTT inner loops of mini-batches of 32, 48 or 64 tokens on 64-wide heads (and
+// TTT inner loops of mini-batches of 16 to 64 tokens on 64-wide heads (and
 // of the 32-wide MLP with 128 hidden units): one workgroup holds a whole
 // mini-batch in LDS and every product is 16 x 16 output tiles of fp32 MFMA,
 // one K x 64 tile per wave.
@@ -24,6 +24,11 @@
 // The shapes taken are those that a layer (FF = F) or the 4x MLP builds of
 // 32- and 64-wide heads; others keep the general-shape kernels.
 //
+// Mini-batches of 16 tokens in fp32 run here too where the caller asks for it
+// (the split form, TTT_FORM_SPLIT): one wave per SIMD, so every product's operands
+// are requested together and nothing waits behind a store.  Linear B2 H4, 16
+// mini-batches, inference: 62 us in the specialised kernel, 36 here.
+//
 // Everything is held and summed in fp32 whatever the activation type, as in
 // the general-shape kernels (ttt_generic.hip); activations are converted on
 // load.  `saved` holds one slot per (chain, mini-batch), WideSlot below.
@@ -45,10 +50,13 @@ template <int KT_, int FT_, int NSL_, bool MLP_> struct WideShape {
   static constexpr int V = F / 16;         // features per thread in a row pass
   static constexpr int TW = FT * 4;        // 16 x 16 tiles of one slice of W1 or W2
   static constexpr int NT = (TW + NW - 1) / NW;  // of those, per wave
+  // whether every wave has a tile in each pass over them (no branch then)
+  static constexpr bool ALLT = TW % NW == 0, ALLF = FT == 4, ALLK = KT == 4;
   // LDS rows are padded by 4 floats: row-major float4 reads (16 rows x 4 lane
   // groups) and column reads (4 rows x 16 lanes) both touch 64 distinct banks
   static constexpr int LS = S + 4, LF = F + 4, LK = K + 4;
   static constexpr int SLOT = 64 * LS;     // one LDS matrix of up to 64 x 64
+  static constexpr int KSLOT = K * LS;     // one of K rows
   static_assert(MLP || (FT == 4 && NSL == 1), "the Linear loop: 64 features, one slice");
 };
 
@@ -103,33 +111,50 @@ struct WideArgs {
 // B[j * LB + k] : B[k * LB + j].  fp32 MFMA with the operands swapped, so that
 // lane (g, r) holds C[r][4g .. 4g + 3]: four consecutive columns of one row
 // (16-byte LDS and global accesses, per-row factors one scalar per lane).
+// Of a single wave per SIMD (K = 16) every operand is requested before the first
+// MFMA: left to itself the compiler waits for each pair of LDS reads in front of
+// its two MFMAs.  (With four waves per SIMD the others' MFMAs cover that, and the
+// batched reads queue: the MLP's state launches at K = F = FF = 64 took 10% more.)
 // With CS, `cs` receives op(B)'s column sums (column r, in every lane group).
-template <int KD, bool TA, bool TB, int LA, int LB, bool CS = false>
+// what may cross: VALU, SALU, VMEM, LDS writes; LDS reads and MFMAs may not
+constexpr int kSchedKeepLdsReads = 0x2 | 0x4 | 0x70 | 0x200;
+template <class C, int KD, bool TA, bool TB, int LA, int LB, bool CS = false>
 __device__ __forceinline__ f4 wmm(f4 c, const float* A, const float* B, float* cs = nullptr) {
   const int l = lane_id(), g = l >> 4, r = l & 15;
   const float* ap = TA ? A + 4 * g * LA + r : A + r * LA + 4 * g;
   const float* bp = TB ? B + r * LB + 4 * g : B + 4 * g * LB + r;
-  float t = 0.f;
+  Frag<float> a[KD / 16], b[KD / 16];
 #pragma unroll
   for (int k = 0; k < KD; k += 16) {
-    Frag<float> a, b;
     if constexpr (TA) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) a.v[j] = ap[(k + j) * LA];
+      for (int j = 0; j < 4; ++j) a[k / 16].v[j] = ap[(k + j) * LA];
     } else {
-      a.v = *reinterpret_cast<const f4*>(ap + k);
+      a[k / 16].v = *reinterpret_cast<const f4*>(ap + k);
     }
     if constexpr (TB) {
-      b.v = *reinterpret_cast<const f4*>(bp + k);
+      b[k / 16].v = *reinterpret_cast<const f4*>(bp + k);
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b.v[j] = bp[(k + j) * LB];
+      for (int j = 0; j < 4; ++j) b[k / 16].v[j] = bp[(k + j) * LB];
     }
-    if constexpr (CS) t += (b.v[0] + b.v[1]) + (b.v[2] + b.v[3]);
-    mma16(c, b, a);
+  }
+  if constexpr (C::KT == 1) __builtin_amdgcn_sched_barrier(kSchedKeepLdsReads);
+  float t = 0.f;
+#pragma unroll
+  for (int k = 0; k < KD / 16; ++k) {
+    if constexpr (CS) t += (b[k].v[0] + b[k].v[1]) + (b[k].v[2] + b[k].v[3]);
+    mma16(c, b[k], a[k]);
   }
   if constexpr (CS) *cs = sum_col4(t);
   return c;
+}
+
+// this wave's index: uniform, below NW
+template <class C> __device__ __forceinline__ int wide_wave() {
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __builtin_assume(w >= 0 && w < C::NW);
+  return w;
 }
 
 // the 16 x 16 tile grid of an R x Cc-tile product over the waves: tile w
@@ -138,6 +163,12 @@ template <int CT> struct WideTile {
   __device__ __forceinline__ explicit WideTile(int t) : it(t / CT), jt(t % CT) {}
   __device__ __forceinline__ int row() const { return 16 * it + (lane_id() & 15); }
   __device__ __forceinline__ int col() const { return 16 * jt + 4 * (lane_id() >> 4); }
+  // this lane's four columns in a matrix of row width LD: the tile's part of the
+  // address is uniform over the wave, the lane's an unsigned offset (global
+  // accesses then take a scalar base and one 32-bit register per row width)
+  template <int LD, class P> __device__ __forceinline__ P* at(P* base) const {
+    return base + (16 * it * LD + 16 * jt) + ((unsigned)(lane_id() & 15) * LD + 4u * (lane_id() >> 4));
+  }
 };
 
 // ---------------------------------------------------------------- loads, stores
@@ -182,12 +213,21 @@ template <typename T, int V> __device__ __forceinline__ void stact(T* p, typenam
   *reinterpret_cast<typename VecT<T, V>::type*>(p) = y;
 }
 
-// eta[K - 1][j] of a mini-batch whose eta (lr) starts at row0 = slot * K
-template <typename T, int K> __device__ __forceinline__ float wide_eta_last(const WideArgs& a, size_t slot, int j) {
-  if (a.eta_rule == TTT_ETA_DENSE) return (float)static_cast<const T*>(a.eta)[(slot * K + (K - 1)) * K + j];
-  const float* e = static_cast<const float*>(a.eta);
-  if (a.eta_rule == TTT_ETA_DENSE_F32) return e[(slot * K + (K - 1)) * K + j];
-  return e[slot * K + j] * (1.0f / (float)K);
+// eta[K - 1][j] of a mini-batch whose eta (lr) starts at row0 = slot * K: as
+// loaded, so that a request made ahead is not waited for where it is made ...
+template <typename T, int K> __device__ __forceinline__ unsigned wide_eta_last_raw(const WideArgs& a, size_t slot, int j) {
+  const size_t last = (slot * K + (K - 1)) * K + j;
+  if constexpr (sizeof(T) == 2)
+    if (a.eta_rule == TTT_ETA_DENSE) return static_cast<const unsigned short*>(a.eta)[last];
+  const bool dense = a.eta_rule == TTT_ETA_DENSE || a.eta_rule == TTT_ETA_DENSE_F32;
+  return static_cast<const unsigned*>(a.eta)[dense ? last : slot * K + j];
+}
+// ... and its value
+template <typename T, int K> __device__ __forceinline__ float wide_eta_last_val(const WideArgs& a, unsigned raw) {
+  if constexpr (sizeof(T) == 2)
+    if (a.eta_rule == TTT_ETA_DENSE) return (float)__builtin_bit_cast(T, (unsigned short)raw);
+  const float e = __builtin_bit_cast(float, raw);
+  return a.eta_rule == TTT_ETA_LAYER || a.eta_rule == TTT_ETA_CAUSAL ? e * (1.0f / (float)K) : e;
 }
 // eta[i][j .. j + 3]
 template <typename T, int K> __device__ __forceinline__ f4 wide_eta4(const WideArgs& a, size_t slot, int i, int j) {

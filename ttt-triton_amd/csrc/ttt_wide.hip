@@ -9,7 +9,8 @@ namespace {
 template <int KT, typename Fn> size_t wide_visit_kt(int F, int FF, bool mlp, Fn f) {
   if (!mlp) return F == 64 ? f(WideShape<KT, 4, 1, false>{}) : 0;
   if (F == 64 && FF == 64) return f(WideShape<KT, 4, 1, true>{});
-  if (F == 64 && FF == 256) return f(WideShape<KT, 4, 4, true>{});
+  if constexpr (KT > 1)
+    if (F == 64 && FF == 256) return f(WideShape<KT, 4, 4, true>{});
   if (F == 32 && FF == 128) return f(WideShape<KT, 2, 2, true>{});
   return 0;
 }
@@ -18,6 +19,7 @@ template <int KT, typename Fn> size_t wide_visit_kt(int F, int FF, bool mlp, Fn 
 size_t wide_slot_bytes(int K, int F, int FF, bool mlp) {
   auto bytes = [](auto shape) { return WideSlot<decltype(shape)>::FLOATS * sizeof(float); };
   switch (K) {
+    case 16: return wide_visit_kt<1>(F, FF, mlp, bytes);
     case 32: return wide_visit_kt<2>(F, FF, mlp, bytes);
     case 48: return wide_visit_kt<3>(F, FF, mlp, bytes);
     case 64: return wide_visit_kt<4>(F, FF, mlp, bytes);
@@ -35,7 +37,8 @@ hipError_t launch_wide(const WideArgs& a, int B, int K, int F, int FF, bool mlp,
 
 }  // namespace
 
-bool wide_shape_ok(int K, int F, int FF, bool mlp) { return wide_slot_bytes(K, F, FF, mlp) != 0; }
+// (16-token mini-batches only where the caller asks for the split form)
+bool wide_shape_ok(int K, int F, int FF, bool mlp) { return K > 16 && wide_slot_bytes(K, F, FF, mlp) != 0; }
 
 size_t wide_saved_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp) {
   return (size_t)B * H * NC * wide_slot_bytes(K, F, FF, mlp);

@@ -24,7 +24,8 @@ template <typename T, int KT> hipError_t wide_kt(const WideArgs& a, int F, int F
              : wide_fwd<T, WideShape<KT, FT, NSL, MLP>>(a, chains, stream)
   if (!mlp) TTT_WIDE(4, 1, false);
   if (F == 64 && FF == 64) TTT_WIDE(4, 1, true);
-  if (F == 64 && FF == 256) TTT_WIDE(4, 4, true);
+  if constexpr (KT > 1)
+    if (F == 64 && FF == 256) TTT_WIDE(4, 4, true);
   if (F == 32 && FF == 128) TTT_WIDE(2, 2, true);
 #undef TTT_WIDE
   return hipErrorInvalidValue;
@@ -35,6 +36,9 @@ template <typename T, int KT> hipError_t wide_kt(const WideArgs& a, int F, int F
 template <typename T>
 hipError_t launch_wide_t(const WideArgs& a, int K, int F, int FF, bool mlp, bool bwd, int chains, hipStream_t stream) {
   switch (K) {
+    case 16:
+      if constexpr (sizeof(T) == 4) return wide_kt<T, 1>(a, F, FF, mlp, bwd, chains, stream);
+      return hipErrorInvalidValue;
     case 32: return wide_kt<T, 2>(a, F, FF, mlp, bwd, chains, stream);
     case 48: return wide_kt<T, 3>(a, F, FF, mlp, bwd, chains, stream);
     case 64: return wide_kt<T, 4>(a, F, FF, mlp, bwd, chains, stream);

@@ -9,6 +9,8 @@ import ctypes
 import os
 import threading
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # TTT_AMD_LIB names another build of the same library (e.g. the host-ASan
 # checking build of build_lib.py --asan)
@@ -25,6 +27,7 @@ ETA_DENSE = 0
 ETA_LAYER = 1
 ETA_CAUSAL = 2
 ETA_DENSE_F32 = 3  # dense eta kept in fp32 under 16-bit activations (chosen from eta's dtype)
+FORM_SPLIT = 0x100  # or'ed into the eta rule: the state and the readout as two launches
 ETA_RULES = {"dense": ETA_DENSE, "layer": ETA_LAYER, "causal": ETA_CAUSAL}
 
 # process-wide options (enum ttt_option)
@@ -50,6 +53,7 @@ SIGNATURES = {
     "ttt_linear_bwd": (_I, [_P] * 9 + [_I] * 8 + [_F] + [_P] * 8 + [_P, _S, _P]),
     "ttt_mlp_fwd": (_I, [_P] * 10 + [_I] * 10 + [_F] + [_P] * 13 + [_P, _S, _P]),
     "ttt_mlp_saved_bytes": (_S, [_I] * 7),
+    "ttt_split_saved_bytes": (_S, [_I] * 6),
     "ttt_mlp_bwd_workspace_bytes": (_S, [_I] * 7),
     "ttt_mlp_bwd": (_I, [_P] * 15 + [_I] * 9 + [_F] + [_P] * 10 + [_P, _S, _P, _S, _P]),
     "ttt_mlp_bwd_noalloc": (_I, [_P] * 15 + [_I] * 9 + [_F] + [_P] * 10 + [_P, _S, _P]),
@@ -113,6 +117,26 @@ def fast_linear_shape(K: int, F: int) -> bool:
 
 def fast_mlp_shape(K: int, F: int, FF: int) -> bool:
     return fast_linear_shape(K, F) and FF in (64, 128, 256)
+
+
+# The split form's `saved` buffer is bounded: it holds every mini-batch's state.
+SPLIT_MAX_BYTES = 1 << 30
+
+
+def split_form(XQ, FF: int) -> bool:
+    """Whether 16-token mini-batches in fp32 run the split form (FORM_SPLIT; FF = 0:
+    the Linear loop).  One chain is one workgroup of the specialised kernels,
+    whose readout shares that workgroup's time with the recurrence; the split
+    form runs it on the rest of the GPU, and loses once the chains fill that.
+    Kernel times specialised / split, 32 mini-batches, forward + backward at
+    8, 64, 128 (96) chains: Linear 342/195, 348/239, 353/338 us (192 chains:
+    359/415); MLP F = FF = 64 547/378, 559/474, (579/581); F = 32, FF = 128
+    734/479, 741/584, (758/705).  In 16 bits the specialised kernels' shorter
+    products win at every count (Linear 120/198 at 8 chains), and at F = 64,
+    FF = 256 in fp32 (1239/1505)."""
+    if XQ.dim() != 5 or XQ.dtype != torch.float32 or XQ.shape[0] * XQ.shape[1] > (64 if FF else 128):
+        return False
+    return 0 < load().ttt_split_saved_bytes(*XQ.shape, FF) <= SPLIT_MAX_BYTES
 
 
 def eta_rule_code(rule) -> int:

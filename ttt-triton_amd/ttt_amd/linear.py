@@ -41,7 +41,7 @@ def _check_shapes(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, rule=_lib.ETA_DENSE):
 
 def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_EPS,
                    want_ckpt: bool = True, want_last: bool = False, want_saved: bool = False,
-                   eta_rule="dense"):
+                   eta_rule="dense", split: bool = False):
     """Run the forward kernel.  `eta` is the dense [B,H,NC,K,K] tensor
     (eta_rule "dense") or the learning rates lr [B,H,NC,K] expanded on chip
     by eta_rule "layer" or "causal".  Returns (out [B,H,NC,K,F] in XQ.dtype,
@@ -49,7 +49,10 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
 
     `saved` (uint8, ttt_linear_saved_bytes long) holds what linear_backward
     reads instead of re-running the forward; the backward needs it together
-    with W1_ckpt and W1_last."""
+    with W1_ckpt and W1_last.  With `split` (fp32, K = 16, F = 64) the state and the
+    readout run as two launches (TTT_FORM_SPLIT): the buffer is then
+    ttt_split_saved_bytes long, always allocated, and all that a split backward
+    needs."""
     rule = _lib.eta_rule_code(eta_rule)
     B, H, NC, K, F = _check_shapes(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, rule)
     dev = check_device(XQ, XK, XV, eta, W1, b1, ln_w, ln_b)
@@ -73,8 +76,11 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
                 torch.empty((B, H, 1, F), device=dev, dtype=torch.float32))
     lib = _lib.load()
     saved = None
-    if want_saved or not _lib.fast_linear_shape(K, F):
-        nbytes = lib.ttt_linear_saved_bytes(B, H, NC, K, F)
+    if split:
+        krule |= _lib.FORM_SPLIT
+    if want_saved or split or not _lib.fast_linear_shape(K, F):
+        nbytes = (lib.ttt_split_saved_bytes(B, H, NC, K, F, 0) if split
+                  else lib.ttt_linear_saved_bytes(B, H, NC, K, F))
         saved = torch.empty(nbytes, device=dev, dtype=torch.uint8)
     with torch.cuda.device(dev):
         st = lib.ttt_linear_fwd(
@@ -89,20 +95,23 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
 
 
 def linear_backward(ln_w, ln_b, XQ, XV, XK, eta, W1_ckpt, W1_last, saved, dout, G: int, eps: float = LN_EPS,
-                    eta_rule="dense", sum_ln: bool = True):
+                    eta_rule="dense", sum_ln: bool = True, split: bool = False):
     """Run the backward kernel on what linear_forward(want_ckpt, want_last,
     want_saved) returned.  Returns fp32 (dln_w [H,F], dln_b [H,F],
     dW1 [B,H,F,F], db1 [B,H,1,F]) and (dXQ, dXV, dXK, deta) in XQ.dtype,
     deta being dlr [B,H,NC,K] fp32 for an lr eta rule, and fp32 for a dense
     fp32 eta under 16-bit activations (read in fp32 too).  With sum_ln=False
-    dln_w and dln_b are the per-chain partials [B,H,F]."""
+    dln_w and dln_b are the per-chain partials [B,H,F].  `split` as in the
+    forward; W1_ckpt and W1_last are then not read and may be None."""
     rule = _lib.eta_rule_code(eta_rule)
     B, H, NC, K, F = XQ.shape
-    dev = check_device(XQ, XK, XV, eta, W1_ckpt, W1_last, saved, dout)
+    dev = check_device(XQ, XK, XV, eta, saved, dout, *(t for t in (W1_ckpt, W1_last) if t is not None))
     mp = XQ.dtype
     code = dtype_code(mp)
     xq, xk, xv, do = (as_act(t, mp) for t in (XQ, XK, XV, dout))
     et, krule = eta_operand(eta, rule, mp)
+    if split:
+        krule |= _lib.FORM_SPLIT
     lw = ln_w.detach().to(torch.float32).contiguous()
     lb = ln_b.detach().to(torch.float32).contiguous()
     dxq = torch.empty_like(xq)
@@ -116,7 +125,8 @@ def linear_backward(ln_w, ln_b, XQ, XV, XK, eta, W1_ckpt, W1_last, saved, dout, 
     lib = _lib.load()
     with torch.cuda.device(dev):
         st = lib.ttt_linear_bwd(
-            ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb), ptr(W1_ckpt), ptr(W1_last), ptr(do),
+            ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb),
+            *(ptr(t) if t is not None else None for t in (W1_ckpt, W1_last)), ptr(do),
             B, H, NC, K, F, int(G), code, krule, float(eps),
             ptr(dxq), ptr(dxk), ptr(dxv), ptr(deta), ptr(dW), ptr(db), ptr(dlw), ptr(dlb),
             ptr(saved), saved.numel(), stream_of(dev))
@@ -139,13 +149,15 @@ class TTTLinearFunction(torch.autograd.Function):
         G = min(max(int(checkpoint_group_size), 1), NC)
         # what the backward reads only when a gradient is wanted
         train = any(ctx.needs_input_grad)
+        split = _lib.split_form(XQ_batch, 0)
         out, ck, last, saved = linear_forward(ttt_norm_weight, ttt_norm_bias, W1_init, b1_init, XQ_batch,
-                                              XV_batch, XK_batch, eta_batch, G, eps, want_ckpt=train,
-                                              want_last=train, want_saved=train, eta_rule=eta_rule)
+                                              XV_batch, XK_batch, eta_batch, G, eps, want_ckpt=train and not split,
+                                              want_last=train and not split, want_saved=train, eta_rule=eta_rule,
+                                              split=split)
         if train:
-            ctx.save_for_backward(XQ_batch, XV_batch, XK_batch, eta_batch, ttt_norm_weight, ttt_norm_bias, ck[0],
-                                  last[0], saved)
-        ctx.G, ctx.eps, ctx.eta_rule = G, eps, eta_rule
+            ctx.save_for_backward(XQ_batch, XV_batch, XK_batch, eta_batch, ttt_norm_weight, ttt_norm_bias,
+                                  *((None, None) if split else (ck[0], last[0])), saved)
+        ctx.G, ctx.eps, ctx.eta_rule, ctx.split = G, eps, eta_rule, split
         ctx.dtypes = (ttt_norm_weight.dtype, ttt_norm_bias.dtype, W1_init.dtype, b1_init.dtype,
                       XQ_batch.dtype, XV_batch.dtype, XK_batch.dtype, eta_batch.dtype)
         return out
@@ -154,7 +166,8 @@ class TTTLinearFunction(torch.autograd.Function):
     def backward(ctx, grad_out):
         XQ, XV, XK, eta, lw, lb, Wc, Wl, saved = ctx.saved_tensors
         (dlw, dlb, dW, db), (dxq, dxv, dxk, deta) = linear_backward(
-            lw, lb, XQ, XV, XK, eta, Wc, Wl, saved, grad_out, ctx.G, ctx.eps, eta_rule=ctx.eta_rule)
+            lw, lb, XQ, XV, XK, eta, Wc, Wl, saved, grad_out, ctx.G, ctx.eps, eta_rule=ctx.eta_rule,
+            split=ctx.split)
         grads = (dlw, dlb, dW, db, dxq, dxv, dxk, deta)
         grads = tuple(gr.to(dt) for gr, dt in zip(grads, ctx.dtypes))
         return grads + (None, None, None)

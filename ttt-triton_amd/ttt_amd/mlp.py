@@ -57,7 +57,7 @@ def _check_shapes(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, rule=_lib.ETA_DEN
 
 def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0, eps: float = LN_EPS,
                 want_ckpt: bool = True, want_last: bool = False, want_saved: bool = False,
-                ckpt_w1_only: bool = False, eta_rule="dense"):
+                ckpt_w1_only: bool = False, eta_rule="dense", split: bool = False):
     """Run the forward kernel.  `eta` is the dense [B,H,NC,K,K] tensor
     (eta_rule "dense") or the learning rates lr [B,H,NC,K] that the kernel
     expands by eta_rule "layer" (lr[j]/K in every row) or "causal"
@@ -67,7 +67,11 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     checkpoints every G mini-batches, the final state, and each mini-batch's
     state-update operands and activations (a flat uint8 buffer of
     ttt_mlp_saved_bytes).  The backward reads only W1's checkpoints: with
-    ckpt_w1_only the other three are neither allocated nor written (None)."""
+    ckpt_w1_only the other three are neither allocated nor written (None).
+    With `split` (fp32, K = 16; F = FF = 64, or F = 32 with FF = 128)
+    the state and the readout run as two launches (TTT_FORM_SPLIT): the saved
+    buffer is then ttt_split_saved_bytes long, always allocated, and all that a
+    split backward needs."""
     rule = _lib.eta_rule_code(eta_rule)
     B, H, NC, K, F, FF = _check_shapes(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, rule)
     dev = check_device(XQ, XK, XV, eta, W1, b1, W2, b2, ln_w, ln_b)
@@ -95,8 +99,12 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     none4 = (None, None, None, None)
     lib = _lib.load()
     saved = None
-    if want_saved or not _lib.fast_mlp_shape(K, F, FF):
-        saved = torch.empty(lib.ttt_mlp_saved_bytes(B, H, NC, K, F, FF, code), device=dev, dtype=torch.uint8)
+    if split:
+        krule |= _lib.FORM_SPLIT
+    if want_saved or split or not _lib.fast_mlp_shape(K, F, FF):
+        nbytes = (lib.ttt_split_saved_bytes(B, H, NC, K, F, FF) if split
+                  else lib.ttt_mlp_saved_bytes(B, H, NC, K, F, FF, code))
+        saved = torch.empty(nbytes, device=dev, dtype=torch.uint8)
     with torch.cuda.device(dev):
         st = lib.ttt_mlp_fwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb), ptr(w1), ptr(bb1), ptr(w2), ptr(bb2),
@@ -111,7 +119,7 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
 
 
 def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, eps: float = LN_EPS,
-                 workspace=None, eta_rule="dense", check_timeout=None, sum_ln: bool = True):
+                 workspace=None, eta_rule="dense", check_timeout=None, sum_ln: bool = True, FF: int = 0):
     """Run the backward kernel.  ckpt = (W1, b1, W2, b2) checkpoints, last =
     the final state and saved = the saved buffer, all from one mlp_forward
     call with the same G and eta form.  `workspace` (uint8, at least
@@ -123,15 +131,20 @@ def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, e
     fp32 for a dense fp32 eta under 16-bit activations (read in fp32 too).
     With check_timeout (default: TTT_AMD_CHECK set) the call waits for the
     launch and raises TTTError if a fused dXQ/dXK worker gave up waiting.
-    With sum_ln=False dln_w and dln_b are the per-chain partials [B,H,F]."""
+    With sum_ln=False dln_w and dln_b are the per-chain partials [B,H,F].
+    `saved` of a split forward: ckpt = last = None, FF the hidden width."""
     rule = _lib.eta_rule_code(eta_rule)
     B, H, NC, K, F = XQ.shape
-    FF = ckpt[0].shape[-1]
-    dev = check_device(XQ, XK, XV, eta, dout, *(t for t in ckpt if t is not None), *last, saved)
+    split = ckpt is None
+    ckpt, last = ckpt or (None,) * 4, last or (None,) * 4
+    FF = FF if split else ckpt[0].shape[-1]
+    dev = check_device(XQ, XK, XV, eta, dout, *(t for t in (*ckpt, *last) if t is not None), saved)
     mp = XQ.dtype
     code = dtype_code(mp)
     xq, xk, xv, do = (as_act(t, mp) for t in (XQ, XK, XV, dout))
     et, krule = eta_operand(eta, rule, mp)
+    if split:
+        krule |= _lib.FORM_SPLIT
     lw, lb = _f32(ln_w), _f32(ln_b)
     dxq, dxk, dxv = torch.empty_like(xq), torch.empty_like(xq), torch.empty_like(xq)
     deta = torch.empty_like(et)
@@ -140,18 +153,17 @@ def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, e
     dW2, db2 = torch.empty((B, H, FF, F), **f32), torch.empty((B, H, 1, F), **f32)
     dlw, dlb = torch.empty((B, H, F), **f32), torch.empty((B, H, F), **f32)
     lib = _lib.load()
-    nws = lib.ttt_mlp_bwd_workspace_bytes(B, H, NC, K, F, FF, code)
+    nws = 0 if split else lib.ttt_mlp_bwd_workspace_bytes(B, H, NC, K, F, FF, code)
     ws = torch.empty(nws, device=dev, dtype=torch.uint8) if workspace is None else workspace
     with torch.cuda.device(dev):
         st = lib.ttt_mlp_bwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb),
-            *(ptr(t) if t is not None else None for t in ckpt),
-            *(ptr(t) for t in last), ptr(do),
+            *(ptr(t) if t is not None else None for t in (*ckpt, *last)), ptr(do),
             B, H, NC, K, F, FF, int(G), code, krule, float(eps),
             ptr(dxq), ptr(dxk), ptr(dxv), ptr(deta), ptr(dW1), ptr(db1), ptr(dW2), ptr(db2), ptr(dlw), ptr(dlb),
             ptr(saved), saved.numel(), ptr(ws), ws.numel(), stream_of(dev))
     _lib.check(st, "ttt_mlp_bwd")
-    if CHECK_BWD if check_timeout is None else check_timeout:
+    if not split and (CHECK_BWD if check_timeout is None else check_timeout):
         _lib.check(mlp_bwd_status(ws, B, H, NC, K, F, FF, code), "ttt_mlp_bwd")
     if sum_ln:
         dlw, dlb = dlw.sum(0), dlb.sum(0)
@@ -184,13 +196,16 @@ class TTTMLPFunction(torch.autograd.Function):
         # what the backward reads (checkpoints, final state, saved buffer) only
         # when a gradient is wanted: an inference forward skips those stores
         train = any(ctx.needs_input_grad)
+        split = _lib.split_form(XQ_batch, W1_init.shape[-1])
+        keep = train and not split
         out, ck, memo, last, saved = mlp_forward(ttt_norm_weight, ttt_norm_bias, W1_init, b1_init, W2_init, b2_init,
                                                XQ_batch, XV_batch, XK_batch, eta_batch, G, M=M, eps=eps,
-                                               want_ckpt=train, want_last=train, want_saved=train,
-                                               ckpt_w1_only=True, eta_rule=eta_rule)
+                                               want_ckpt=keep, want_last=keep, want_saved=train,
+                                               ckpt_w1_only=True, eta_rule=eta_rule, split=split)
         if train:
-            ctx.save_for_backward(XQ_batch, XV_batch, XK_batch, eta_batch, ttt_norm_weight, ttt_norm_bias, *ck,
-                                  *last, saved)
+            ctx.save_for_backward(XQ_batch, XV_batch, XK_batch, eta_batch, ttt_norm_weight, ttt_norm_bias, saved,
+                                  *(() if split else (*ck, *last)))
+        ctx.FF = W1_init.shape[-1]
         ctx.G, ctx.eps, ctx.eta_rule = G, eps, eta_rule
         ctx.dtypes = (ttt_norm_weight.dtype, ttt_norm_bias.dtype, W1_init.dtype, b1_init.dtype, W2_init.dtype,
                       b2_init.dtype, XQ_batch.dtype, XV_batch.dtype, XK_batch.dtype, eta_batch.dtype)
@@ -201,10 +216,10 @@ class TTTMLPFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out, *unused):
-        XQ, XV, XK, eta, lw, lb = ctx.saved_tensors[:6]
-        ck, last, saved = ctx.saved_tensors[6:10], ctx.saved_tensors[10:14], ctx.saved_tensors[14]
+        XQ, XV, XK, eta, lw, lb, saved = ctx.saved_tensors[:7]
+        ck, last = ctx.saved_tensors[7:11] or None, ctx.saved_tensors[11:15] or None
         (dlw, dlb, dW1, db1, dW2, db2), (dxq, dxv, dxk, deta) = mlp_backward(
-            lw, lb, XQ, XV, XK, eta, ck, last, saved, grad_out, ctx.G, ctx.eps, eta_rule=ctx.eta_rule)
+            lw, lb, XQ, XV, XK, eta, ck, last, saved, grad_out, ctx.G, ctx.eps, eta_rule=ctx.eta_rule, FF=ctx.FF)
         grads = (dlw, dlb, dW1, db1, dW2, db2, dxq, dxv, dxk, deta)
         grads = tuple(gr.to(dt) for gr, dt in zip(grads, ctx.dtypes))
         return grads + (None, None, None, None)
