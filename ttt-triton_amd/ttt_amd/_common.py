@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from . import _lib
@@ -19,7 +21,12 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def as_act(t: torch.Tensor, dt: torch.dtype) -> torch.Tensor:
     """Activation in the path's dtype, contiguous (no copy when already so)."""
-    return t.detach().to(dt).contiguous()
+    return t if t.dtype == dt and t.is_contiguous() else t.detach().to(dt).contiguous()
+
+
+def f32c(t: torch.Tensor) -> torch.Tensor:
+    """fp32 and contiguous (no copy when already so)."""
+    return as_act(t, torch.float32)
 
 
 def eta_operand(eta: torch.Tensor, rule: int, dt: torch.dtype):
@@ -30,9 +37,9 @@ def eta_operand(eta: torch.Tensor, rule: int, dt: torch.dtype):
     A learning-rate vector is fp32."""
     if rule == _lib.ETA_DENSE:
         if eta.dtype == torch.float32 and dt != torch.float32:
-            return eta.detach().contiguous(), _lib.ETA_DENSE_F32
+            return f32c(eta), _lib.ETA_DENSE_F32
         return as_act(eta, dt), rule
-    return eta.detach().to(torch.float32).contiguous(), rule
+    return f32c(eta), rule
 
 
 def check_device(*ts: torch.Tensor) -> torch.device:
@@ -43,6 +50,19 @@ def check_device(*ts: torch.Tensor) -> torch.device:
         if t.device != dev:
             raise ValueError(f"all tensors must be on {dev}, got {t.device}")
     return dev
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(dev: torch.device):
+    """torch.cuda.device(dev), free where dev is the current device already."""
+    return _HERE if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
+def grads_as(grads, dtypes):
+    """Each gradient in its input's type."""
+    return tuple(g if g.dtype == dt else g.to(dt) for g, dt in zip(grads, dtypes))
 
 
 def ptr(t: torch.Tensor) -> int:

@@ -15,7 +15,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._common import check_device, dtype_code, ptr, stream_of
+from ._common import as_act, check_device, dtype_code, f32c, grads_as, on_device, ptr, stream_of
 
 RECON_EPS = 1e-8     # ttt_layer.py:230
 POST_NORM_EPS = 1e-6  # ttt_layer.py:78
@@ -71,13 +71,13 @@ class ProducerFunction(torch.autograd.Function):
         dev = check_device(proj, rope, ln_w, ln_b)
         code = dtype_code(proj.dtype)
         pj = proj.contiguous()
-        rp = rope.to(torch.float32).contiguous()
-        lw, lb = ln_w.detach().to(torch.float32).contiguous(), ln_b.detach().to(torch.float32).contiguous()
+        rp = f32c(rope)
+        lw, lb = f32c(ln_w), f32c(ln_b)
         NC = L // K
         outs = [torch.empty((B, H, NC, K, F), device=dev, dtype=proj.dtype) for _ in range(4)]
         lr = torch.empty((B, H, NC, K), device=dev, dtype=torch.float32)
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with on_device(dev):
             st = lib.ttt_qkvu_producer_fwd(ptr(pj), ld, ptr(rp), ptr(lw), ptr(lb), B, L, H, K, F, float(base_lr),
                                            float(eps), code, *(ptr(t) for t in outs), ptr(lr), stream_of(dev))
         _lib.check(st, "ttt_qkvu_producer_fwd")
@@ -96,21 +96,20 @@ class ProducerFunction(torch.autograd.Function):
         def act(g):
             if g is None:
                 return torch.zeros((B, H, L // K, K, F), device=dev, dtype=pj.dtype)
-            return g.to(pj.dtype).contiguous()
+            return as_act(g, pj.dtype)
 
         gq, gk, gv, gu = (act(g) for g in (dXQ, dXK, dXV, dXU))
-        gl = dlr.to(torch.float32).contiguous() if dlr is not None else None
+        gl = f32c(dlr) if dlr is not None else None
         dproj = torch.empty_like(pj)
         lib = _lib.load()
         part = torch.empty(lib.ttt_layer_io_partial_bytes(B, L, H, F) // 4, device=dev, dtype=torch.float32)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             st = lib.ttt_qkvu_producer_bwd(ptr(pj), ld, ptr(rp), ptr(lw), ptr(lb), ptr(gq), ptr(gk), ptr(gv), ptr(gu),
                                            ptr(gl) if gl is not None else None, B, L, H, K, F, ctx.base_lr, ctx.eps,
                                            code, ptr(dproj), ptr(part), part.numel() * 4, stream_of(dev))
         _lib.check(st, "ttt_qkvu_producer_bwd")
         dw, db = _partial_sum(part, H * F)
-        return (dproj, None, dw.view(H, F).to(ctx.dtypes[0]), db.view(H, F).to(ctx.dtypes[1]), None, None, None,
-                None)
+        return (dproj, None) + grads_as((dw.view(H, F), db.view(H, F)), ctx.dtypes) + (None,) * 4
 
 
 class PostNormFunction(torch.autograd.Function):
@@ -129,11 +128,11 @@ class PostNormFunction(torch.autograd.Function):
         dev = check_device(XQW, gamma, beta)
         code = dtype_code(XQW.dtype)
         x = XQW.contiguous()
-        g, b = gamma.detach().to(torch.float32).contiguous(), beta.detach().to(torch.float32).contiguous()
+        g, b = f32c(gamma), f32c(beta)
         out = torch.empty((B, L, D), device=dev, dtype=XQW.dtype)
         stats = torch.empty((B * L, 2), device=dev, dtype=torch.float32)
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with on_device(dev):
             st = lib.ttt_post_norm_fwd(ptr(x), ptr(g), ptr(b), B, L, H, K, F, float(eps), code, ptr(out), ptr(stats),
                                        stream_of(dev))
         _lib.check(st, "ttt_post_norm_fwd")
@@ -149,16 +148,16 @@ class PostNormFunction(torch.autograd.Function):
         D, L = H * F, NC * K
         dev = x.device
         code = dtype_code(x.dtype)
-        do = dout.to(x.dtype).contiguous()
+        do = as_act(dout, x.dtype)
         dx = torch.empty_like(x)
         lib = _lib.load()
         part = torch.empty(lib.ttt_layer_io_partial_bytes(B, L, H, F) // 4, device=dev, dtype=torch.float32)
-        with torch.cuda.device(dev):
+        with on_device(dev):
             st = lib.ttt_post_norm_bwd(ptr(x), ptr(g), ptr(stats), ptr(do), B, L, H, K, F, code, ptr(dx), ptr(part),
                                        part.numel() * 4, stream_of(dev))
         _lib.check(st, "ttt_post_norm_bwd")
         dg, db = _partial_sum(part, D)
-        return dx, dg.to(ctx.dtypes[0]), db.to(ctx.dtypes[1]), None
+        return (dx,) + grads_as((dg, db), ctx.dtypes) + (None,)
 
 
 __all__ = ["ProducerFunction", "PostNormFunction", "rope_table", "RECON_EPS", "POST_NORM_EPS"]

@@ -14,7 +14,7 @@ import math
 import torch
 
 from . import _lib
-from ._common import as_act, check_device, dtype_code, eta_operand, ptr, stream_of
+from ._common import as_act, check_device, dtype_code, eta_operand, f32c, grads_as, on_device, ptr, stream_of
 
 LN_EPS = 1e-8  # ops/ttt_utils.py:4,21
 
@@ -62,10 +62,10 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
     NK = math.ceil(NC / G)
     xq, xk, xv = (as_act(t, mp) for t in (XQ, XK, XV))
     et, krule = eta_operand(eta, rule, mp)
-    w1 = W1.detach().to(torch.float32).contiguous()
-    bb = b1.detach().to(torch.float32).contiguous()
-    lw = ln_w.detach().to(torch.float32).contiguous()
-    lb = ln_b.detach().to(torch.float32).contiguous()
+    w1 = f32c(W1)
+    bb = f32c(b1)
+    lw = f32c(ln_w)
+    lb = f32c(ln_b)
     out = torch.empty((B, H, NC, K, F), device=dev, dtype=mp)
     ck = last = None
     if want_ckpt:
@@ -82,7 +82,7 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
         nbytes = (lib.ttt_split_saved_bytes(B, H, NC, K, F, 0) if split
                   else lib.ttt_linear_saved_bytes(B, H, NC, K, F))
         saved = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_linear_fwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb), ptr(w1), ptr(bb),
             B, H, NC, K, F, G, code, krule, float(eps), ptr(out),
@@ -112,18 +112,18 @@ def linear_backward(ln_w, ln_b, XQ, XV, XK, eta, W1_ckpt, W1_last, saved, dout, 
     et, krule = eta_operand(eta, rule, mp)
     if split:
         krule |= _lib.FORM_SPLIT
-    lw = ln_w.detach().to(torch.float32).contiguous()
-    lb = ln_b.detach().to(torch.float32).contiguous()
+    lw = f32c(ln_w)
+    lb = f32c(ln_b)
     dxq = torch.empty_like(xq)
     dxk = torch.empty_like(xq)
     dxv = torch.empty_like(xq)
     deta = torch.empty_like(et)
     dW = torch.empty((B, H, F, F), device=dev, dtype=torch.float32)
     db = torch.empty((B, H, 1, F), device=dev, dtype=torch.float32)
-    dlw = torch.empty((B, H, F), device=dev, dtype=torch.float32)
-    dlb = torch.empty((B, H, F), device=dev, dtype=torch.float32)
+    dln = torch.empty((2, B, H, F), device=dev, dtype=torch.float32)
+    dlw, dlb = dln
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_linear_bwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb),
             *(ptr(t) if t is not None else None for t in (W1_ckpt, W1_last)), ptr(do),
@@ -132,7 +132,7 @@ def linear_backward(ln_w, ln_b, XQ, XV, XK, eta, W1_ckpt, W1_last, saved, dout, 
             ptr(saved), saved.numel(), stream_of(dev))
     _lib.check(st, "ttt_linear_bwd")
     if sum_ln:
-        dlw, dlb = dlw.sum(0), dlb.sum(0)
+        dlw, dlb = dln.sum(1)
     return (dlw, dlb, dW, db), (dxq, dxv, dxk, deta)
 
 
@@ -168,6 +168,4 @@ class TTTLinearFunction(torch.autograd.Function):
         (dlw, dlb, dW, db), (dxq, dxv, dxk, deta) = linear_backward(
             lw, lb, XQ, XV, XK, eta, Wc, Wl, saved, grad_out, ctx.G, ctx.eps, eta_rule=ctx.eta_rule,
             split=ctx.split)
-        grads = (dlw, dlb, dW, db, dxq, dxv, dxk, deta)
-        grads = tuple(gr.to(dt) for gr, dt in zip(grads, ctx.dtypes))
-        return grads + (None, None, None)
+        return grads_as((dlw, dlb, dW, db, dxq, dxv, dxk, deta), ctx.dtypes) + (None, None, None)

@@ -27,7 +27,7 @@ import math
 import torch
 
 from . import _lib
-from ._common import as_act, check_device, dtype_code, ptr, stream_of
+from ._common import as_act, check_device, dtype_code, f32c, grads_as, on_device, ptr, stream_of
 
 READOUT_EPS = 1e-6  # kernels/mlp_cached_readout.py:98
 
@@ -54,10 +54,6 @@ def _check(XQ, XK, XU, XQW, W1, b1, W2, b2, ln_w, ln_b, M):
     return B, H, NC, K, F, FF, M
 
 
-def _f32(t):
-    return t.detach().to(torch.float32).contiguous()
-
-
 def memo_combine_forward(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M: int,
                          eps: float = READOUT_EPS, images: bool = True):
     """Run the combiner.  Returns (out [B,H,NC,K,F] in XQW.dtype, gates) where
@@ -71,15 +67,15 @@ def memo_combine_forward(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln
     mp = XQW.dtype
     code = dtype_code(mp)
     xq, xk, xu, xqw = (as_act(t, mp) for t in (XQ, XK, XU, XQW))
-    ws = [_f32(t) for t in (W1_memo, b1_memo, W2_memo, b2_memo)]
-    lw, lb = _f32(ln_w), _f32(ln_b)
+    ws = [f32c(t) for t in (W1_memo, b1_memo, W2_memo, b2_memo)]
+    lw, lb = f32c(ln_w), f32c(ln_b)
     lib = _lib.load()
     # the gates and, for bf16, the memo states' LDS images that both calls copy in
     nbytes = (lib.ttt_mlp_memo_workspace_bytes(B, H, NC, K, F, FF, M, code) if images
               else lib.ttt_mlp_memo_gates_bytes(B, H, NC, K, F, M))
     gates = torch.empty(nbytes, device=dev, dtype=torch.uint8)
     out = torch.empty((B, H, NC, K, F), device=dev, dtype=mp)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_mlp_memo_combine(ptr(xq), ptr(xk), ptr(xu), ptr(xqw), *(ptr(t) for t in ws), ptr(lw), ptr(lb),
                                       B, H, NC, K, F, FF, M, code, float(eps), ptr(out), ptr(gates), gates.numel(),
                                       stream_of(dev))
@@ -96,11 +92,11 @@ def memo_combine_backward(XQ, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w,
     mp = XQW.dtype
     code = dtype_code(mp)
     xq, xu, xqw, do = (as_act(t, mp) for t in (XQ, XU, XQW, dout))
-    ws = [_f32(t) for t in (W1_memo, b1_memo, W2_memo, b2_memo)]
-    lw, lb = _f32(ln_w), _f32(ln_b)
+    ws = [f32c(t) for t in (W1_memo, b1_memo, W2_memo, b2_memo)]
+    lw, lb = f32c(ln_w), f32c(ln_b)
     dxk, dxu, dxqw = (torch.empty((B, H, NC, K, F), device=dev, dtype=mp) for _ in range(3))
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_mlp_memo_combine_bwd(ptr(xq), ptr(xu), ptr(xqw), *(ptr(t) for t in ws), ptr(lw), ptr(lb),
                                           ptr(do), B, H, NC, K, F, FF, int(M), code, float(eps), ptr(gates),
                                           gates.numel(), ptr(dxk), ptr(dxu), ptr(dxqw), stream_of(dev))
@@ -127,7 +123,7 @@ class MemoCombineFunction(torch.autograd.Function):
     def backward(ctx, dout):
         XQ, XU, XQW, W1, b1, W2, b2, lw, lb, gates = ctx.saved_tensors
         dxk, dxu, dxqw = memo_combine_backward(XQ, XU, XQW, W1, b1, W2, b2, lw, lb, ctx.M, gates, dout, ctx.eps)
-        return (None, dxk.to(ctx.dtypes[0]), dxu.to(ctx.dtypes[1]), dxqw.to(ctx.dtypes[2])) + (None,) * 8
+        return (None,) + grads_as((dxk, dxu, dxqw), ctx.dtypes) + (None,) * 8
 
 
 def mlp_memo_combine(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M: int):

@@ -16,17 +16,13 @@ import os
 import torch
 
 from . import _lib
-from ._common import as_act, check_device, dtype_code, eta_operand, ptr, stream_of
+from ._common import as_act, check_device, dtype_code, eta_operand, f32c, grads_as, on_device, ptr, stream_of
 
 LN_EPS = 1e-8  # ops/ttt_utils.py:4,21
 
 # With TTT_AMD_CHECK=1 every backward waits for its launch and raises if a
 # fused dXQ/dXK worker gave up waiting (its rows are then NaN).
 CHECK_BWD = os.environ.get("TTT_AMD_CHECK", "0") not in ("", "0")
-
-
-def _f32(t):
-    return t.detach().to(torch.float32).contiguous()
 
 
 def _check_shapes(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, rule=_lib.ETA_DENSE):
@@ -81,19 +77,16 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     NK = math.ceil(NC / G)
     xq, xk, xv = (as_act(t, mp) for t in (XQ, XK, XV))
     et, krule = eta_operand(eta, rule, mp)
-    w1, bb1, w2, bb2, lw, lb = (_f32(t) for t in (W1, b1, W2, b2, ln_w, ln_b))
+    w1, bb1, w2, bb2, lw, lb = (f32c(t) for t in (W1, b1, W2, b2, ln_w, ln_b))
     out = torch.empty((B, H, NC, K, F), device=dev, dtype=mp)
 
-    def state(n):
+    def state(n, w1_only=False):
         lead = (B, H) if n is None else (B, H, n)
-        return (torch.empty(lead + (F, FF), device=dev, dtype=torch.float32),
-                torch.empty(lead + (1, FF), device=dev, dtype=torch.float32),
-                torch.empty(lead + (FF, F), device=dev, dtype=torch.float32),
-                torch.empty(lead + (1, F), device=dev, dtype=torch.float32))
+        shapes = ((F, FF),) if w1_only else ((F, FF), (1, FF), (FF, F), (1, F))
+        ts = tuple(torch.empty(lead + s, device=dev, dtype=torch.float32) for s in shapes)
+        return ts + (None,) * (4 - len(ts))
 
-    ck = state(NK) if want_ckpt else None
-    if ck is not None and ckpt_w1_only:
-        ck = (ck[0], None, None, None)
+    ck = state(NK, ckpt_w1_only) if want_ckpt else None
     memo = state(math.ceil(NC / M)) if M and M > 0 else None
     last = state(None) if want_last else None
     none4 = (None, None, None, None)
@@ -105,7 +98,7 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
         nbytes = (lib.ttt_split_saved_bytes(B, H, NC, K, F, FF) if split
                   else lib.ttt_mlp_saved_bytes(B, H, NC, K, F, FF, code))
         saved = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_mlp_fwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb), ptr(w1), ptr(bb1), ptr(w2), ptr(bb2),
             B, H, NC, K, F, FF, G, int(M) if M else 0, code, krule, float(eps), ptr(out),
@@ -145,17 +138,18 @@ def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, e
     et, krule = eta_operand(eta, rule, mp)
     if split:
         krule |= _lib.FORM_SPLIT
-    lw, lb = _f32(ln_w), _f32(ln_b)
+    lw, lb = f32c(ln_w), f32c(ln_b)
     dxq, dxk, dxv = torch.empty_like(xq), torch.empty_like(xq), torch.empty_like(xq)
     deta = torch.empty_like(et)
     f32 = dict(device=dev, dtype=torch.float32)
     dW1, db1 = torch.empty((B, H, F, FF), **f32), torch.empty((B, H, 1, FF), **f32)
     dW2, db2 = torch.empty((B, H, FF, F), **f32), torch.empty((B, H, 1, F), **f32)
-    dlw, dlb = torch.empty((B, H, F), **f32), torch.empty((B, H, F), **f32)
+    dln = torch.empty((2, B, H, F), **f32)
+    dlw, dlb = dln
     lib = _lib.load()
     nws = 0 if split else lib.ttt_mlp_bwd_workspace_bytes(B, H, NC, K, F, FF, code)
     ws = torch.empty(nws, device=dev, dtype=torch.uint8) if workspace is None else workspace
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_mlp_bwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb),
             *(ptr(t) if t is not None else None for t in (*ckpt, *last)), ptr(do),
@@ -166,7 +160,7 @@ def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, e
     if not split and (CHECK_BWD if check_timeout is None else check_timeout):
         _lib.check(mlp_bwd_status(ws, B, H, NC, K, F, FF, code), "ttt_mlp_bwd")
     if sum_ln:
-        dlw, dlb = dlw.sum(0), dlb.sum(0)
+        dlw, dlb = dln.sum(1)
     return (dlw, dlb, dW1, db1, dW2, db2), (dxq, dxv, dxk, deta)
 
 
@@ -174,7 +168,7 @@ def mlp_bwd_status(workspace, B, H, NC, K, F, FF, code) -> int:
     """ttt_mlp_bwd_check on the workspace of the last backward that used it
     (waits for the current stream): 0, or the timeout status."""
     dev = workspace.device
-    with torch.cuda.device(dev):
+    with on_device(dev):
         return _lib.load().ttt_mlp_bwd_check(ptr(workspace), workspace.numel(), B, H, NC, K, F, FF, code,
                                              stream_of(dev))
 
@@ -220,9 +214,7 @@ class TTTMLPFunction(torch.autograd.Function):
         ck, last = ctx.saved_tensors[7:11] or None, ctx.saved_tensors[11:15] or None
         (dlw, dlb, dW1, db1, dW2, db2), (dxq, dxv, dxk, deta) = mlp_backward(
             lw, lb, XQ, XV, XK, eta, ck, last, saved, grad_out, ctx.G, ctx.eps, eta_rule=ctx.eta_rule, FF=ctx.FF)
-        grads = (dlw, dlb, dW1, db1, dW2, db2, dxq, dxv, dxk, deta)
-        grads = tuple(gr.to(dt) for gr, dt in zip(grads, ctx.dtypes))
-        return grads + (None, None, None, None)
+        return grads_as((dlw, dlb, dW1, db1, dW2, db2, dxq, dxv, dxk, deta), ctx.dtypes) + (None, None, None, None)
 
 
 READOUT_EPS = 1e-6  # kernels/mlp_cached_readout.py:98
@@ -268,11 +260,11 @@ def mlp_cached_readout(XQ_seg, W1, b1, W2, b2, ln_w, ln_b, eps: float = READOUT_
         if len(Ss) == 1:
             S = Ss.pop()
     if S is None:
-        ws, S = [_f32(t) for t in ws], 1
-    lw, lb = _f32(ln_w), _f32(ln_b)
+        ws, S = [f32c(t) for t in ws], 1
+    lw, lb = f32c(ln_w), f32c(ln_b)
     out = torch.empty((B, H, NS, K, F), device=dev, dtype=torch.float32)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with on_device(dev):
         st = lib.ttt_mlp_cached_readout(ptr(xq), *(ptr(t) for t in ws), ptr(lw), ptr(lb),
                                         B, H, NS, K, F, FF, int(S), code, float(eps), ptr(out), stream_of(dev))
     _lib.check(st, "ttt_mlp_cached_readout")
