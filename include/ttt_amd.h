@@ -59,9 +59,13 @@ enum ttt_eta_rule { TTT_ETA_DENSE = 0, TTT_ETA_LAYER = 1, TTT_ETA_CAUSAL = 2, TT
  * with TTT_DTYPE_F32 where ttt_split_saved_bytes is not 0: the split form,
  * whose per-chain launch carries the state alone and whose readout (and its
  * gradients) is a second launch with a workgroup per (chain, mini-batch).
- * Faster where few chains leave the GPU idle.  It takes a `saved` buffer of ttt_split_saved_bytes in every call (the backward reads and writes
- * the forward's), no checkpoints, final state or workspace in the backward. */
-enum ttt_form { TTT_FORM_SPLIT = 0x100 };
+ * Faster where few chains leave the GPU idle.  It takes a `saved` buffer of
+ * ttt_split_saved_bytes in every call (the backward reads and writes the
+ * forward's), no checkpoints, final state or workspace in the backward.
+ *
+ * TTT_STATE_SHARED (forwards only): W1_init, b1_init (W2_init, b2_init) are [H,...],
+ * the same for every sequence of the batch, and read in place. */
+enum ttt_form { TTT_FORM_SPLIT = 0x100, TTT_STATE_SHARED = 0x200 };
 
 enum ttt_status {
   TTT_OK = 0,

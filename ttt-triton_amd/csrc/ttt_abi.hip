@@ -29,6 +29,12 @@ bool take_split(int& eta_rule) {
   eta_rule &= ~TTT_FORM_SPLIT;
   return split;
 }
+// the same of TTT_STATE_SHARED: the number of distinct initial states
+int take_states(int& eta_rule, int B, int H) {
+  const bool shared = (eta_rule & TTT_STATE_SHARED) != 0;
+  eta_rule &= ~TTT_STATE_SHARED;
+  return shared ? H : B * H;
+}
 // fp32 dense eta under fp32 activations is the plain dense form
 int eta_rule_of(int r, int dtype) { return r == TTT_ETA_DENSE_F32 && dtype == TTT_DTYPE_F32 ? TTT_ETA_DENSE : r; }
 
@@ -147,6 +153,7 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
   const bool split = take_split(eta_rule);
+  const int NI = take_states(eta_rule, B, H);
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
   eta_rule = eta_rule_of(eta_rule, dtype);
   const bool fast = fast_linear_shape(K, F) && !split;
@@ -185,6 +192,7 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
     q.ln_b = ln_b;
     q.W1_init = W1_init;
     q.b1_init = b1_init;
+    q.NI = NI;
     q.out = out;
     q.W1_last = W1_last;
     q.b1_last = b1_last;
@@ -215,6 +223,7 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
   p.ln_b = ln_b;
   p.W_init = W1_init;
   p.b_init = b1_init;
+  p.NI = NI;
   p.out = out;
   p.W_last = W1_last;
   p.b_last = b1_last;
@@ -339,6 +348,7 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
   const bool split = take_split(eta_rule);
+  const int NI = take_states(eta_rule, B, H);
   const bool fast = fast_mlp_shape(K, F, FF) && !split;
   if (!fast && !ttt::gen_shape_ok(K, F, FF, true)) return TTT_ERR_SHAPE;
   const size_t need =
@@ -388,6 +398,7 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
     q.b1_init = b1_init;
     q.W2_init = W2_init;
     q.b2_init = b2_init;
+    q.NI = NI;
     q.out = out;
     q.W1_last = W1_last;
     q.b1_last = b1_last;
@@ -428,6 +439,7 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
   p.b1_init = b1_init;
   p.W2_init = W2_init;
   p.b2_init = b2_init;
+  p.NI = NI;
   p.out = out;
   p.W1_last = W1_last;
   p.b1_last = b1_last;

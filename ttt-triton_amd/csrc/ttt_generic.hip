@@ -291,6 +291,7 @@ struct GenArgs {
   const void *XQ, *XK, *XV, *eta, *dout;
   const float *ln_w, *ln_b;
   const float *W1_init, *b1_init, *W2_init, *b2_init;
+  int NI;
   void* out;
   StatePtrs last, ckpt, memo;
   void *dXQ, *dXK, *dXV, *deta;
@@ -460,11 +461,12 @@ __global__ __launch_bounds__(kGenThreads) __attribute__((amdgpu_waves_per_eu(1, 
   {
     const State s0 = state_at(0);
     const size_t F = L.F, FF = L.FF;
-    copy_f(s0.W1, a.W1_init + chain * F * FF, F * FF);
-    copy_f(s0.b1, a.b1_init + chain * FF, FF);
+    const size_t ic = chain % (size_t)a.NI;
+    copy_f(s0.W1, a.W1_init + ic * F * FF, F * FF);
+    copy_f(s0.b1, a.b1_init + ic * FF, FF);
     if (L.mlp) {
-      copy_f(s0.W2, a.W2_init + chain * FF * F, FF * F);
-      copy_f(s0.b2, a.b2_init + chain * F, F);
+      copy_f(s0.W2, a.W2_init + ic * FF * F, FF * F);
+      copy_f(s0.b2, a.b2_init + ic * F, F);
     }
   }
   __syncthreads();
@@ -843,6 +845,7 @@ hipError_t launch_gen_fwd(const GenFwdParams& q, int dtype, hipStream_t stream) 
   a.ln_w = q.ln_w;
   a.ln_b = q.ln_b;
   a.W1_init = q.W1_init;
+  a.NI = q.NI;
   a.b1_init = q.b1_init;
   a.W2_init = q.W2_init;
   a.b2_init = q.b2_init;

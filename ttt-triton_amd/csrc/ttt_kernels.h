@@ -11,6 +11,7 @@ namespace ttt {
 struct LinearFwdParams {
   const void *XQ, *XK, *XV, *eta;
   const float *ln_w, *ln_b, *W_init, *b_init;
+  int NI;  // distinct initial states: chain c starts from state c % NI
   void* out;
   float *W_last, *b_last, *W_ckpt, *b_ckpt;
   void* saved;  // per mini-batch values for the backward, LinSavedSlot layout (may be null)
@@ -54,6 +55,7 @@ size_t linear_saved_slot_bytes(int F);
 struct MlpFwdParams {
   const void *XQ, *XK, *XV, *eta;
   const float *ln_w, *ln_b, *W1_init, *b1_init, *W2_init, *b2_init;
+  int NI;  // distinct initial states: chain c starts from state c % NI
   void* out;
   float *W1_last, *b1_last, *W2_last, *b2_last;
   float *W1_ckpt, *b1_ckpt, *W2_ckpt, *b2_ckpt;
@@ -223,6 +225,7 @@ struct GenLayout {
 struct GenFwdParams {
   const void *XQ, *XK, *XV, *eta;
   const float *ln_w, *ln_b, *W1_init, *b1_init, *W2_init, *b2_init;
+  int NI;  // distinct initial states: chain c starts from state c % NI
   void* out;
   float *W1_last, *b1_last, *W2_last, *b2_last;
   float *W1_ckpt, *b1_ckpt, *W2_ckpt, *b2_ckpt;

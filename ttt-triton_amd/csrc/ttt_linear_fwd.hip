@@ -80,11 +80,11 @@ __global__ __launch_bounds__(128) void linear_fwd_kernel(LinearFwdParams p) {
 #pragma unroll
     for (int i = 0; i < FT; ++i)
 #pragma unroll
-      for (int o = 0; o < FT; ++o) W[i][o] = load_tile(p.W_init + (size_t)chain * F * F, F, 16 * i, 16 * o);
+      for (int o = 0; o < FT; ++o) W[i][o] = load_tile(p.W_init + (size_t)(chain % p.NI) * F * F, F, 16 * i, 16 * o);
     float b_tm[FT], lnw_tm[FT], lnb_tm[FT];
 #pragma unroll
     for (int o = 0; o < FT; ++o) {
-      b_tm[o] = p.b_init[(size_t)chain * F + 16 * o + n];
+      b_tm[o] = p.b_init[(size_t)(chain % p.NI) * F + 16 * o + n];
       lnw_tm[o] = p.ln_w[h * F + 16 * o + n];
       lnb_tm[o] = p.ln_b[h * F + 16 * o + n];
     }

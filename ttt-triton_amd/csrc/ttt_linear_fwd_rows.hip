@@ -248,10 +248,10 @@ __device__ __forceinline__ void linear_rows_state(const LinearFwdParams& p, LinR
 #pragma unroll
   for (int i = 0; i < FT; ++i)
 #pragma unroll
-    for (int o = 0; o < FT; ++o) W[i][o] = load_tile(p.W_init + (size_t)chain * F * F, F, 16 * i, 16 * o);
+    for (int o = 0; o < FT; ++o) W[i][o] = load_tile(p.W_init + (size_t)(chain % p.NI) * F * F, F, 16 * i, 16 * o);
   float bn[FT];  // b[16 o + n]
 #pragma unroll
-  for (int o = 0; o < FT; ++o) bn[o] = p.b_init[(size_t)chain * F + 16 * o + n];
+  for (int o = 0; o < FT; ++o) bn[o] = p.b_init[(size_t)(chain % p.NI) * F + 16 * o + n];
 
   Frag<T> xk_cur[FT], xk_nxt[FT], xk_pf[FT];
   ERow er_n;

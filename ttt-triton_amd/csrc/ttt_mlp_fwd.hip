@@ -107,8 +107,9 @@ __global__ __launch_bounds__(64 * NW) void mlp_fwd_kernel(MlpFwdParams p) {
   Tile W1[FT][HT], W2[HT][FT];
   float b1_tm[HT], b2_tm[FT];
   {
-    const rsrc_t r1 = make_rsrc(p.W1_init + (size_t)chain * F * FF, F * FF * 4);
-    const rsrc_t r2 = make_rsrc(p.W2_init + (size_t)chain * FF * F, FF * F * 4);
+    const size_t ic = (size_t)(chain % p.NI);
+    const rsrc_t r1 = make_rsrc(p.W1_init + ic * F * FF, F * FF * 4);
+    const rsrc_t r2 = make_rsrc(p.W2_init + ic * FF * F, FF * F * 4);
 #pragma unroll
     for (int i = 0; i < FT; ++i)
 #pragma unroll
@@ -118,9 +119,9 @@ __global__ __launch_bounds__(64 * NW) void mlp_fwd_kernel(MlpFwdParams p) {
 #pragma unroll
       for (int o = 0; o < FT; ++o) W2[i][o] = bload_tile(r2, w2l, 0, F, 16 * i, 16 * o);
 #pragma unroll
-    for (int o = 0; o < HT; ++o) b1_tm[o] = p.b1_init[(size_t)chain * FF + hs + 16 * o + n];
+    for (int o = 0; o < HT; ++o) b1_tm[o] = p.b1_init[ic * FF + hs + 16 * o + n];
 #pragma unroll
-    for (int o = 0; o < FT; ++o) b2_tm[o] = p.b2_init[(size_t)chain * F + 16 * o + n];
+    for (int o = 0; o < FT; ++o) b2_tm[o] = p.b2_init[ic * F + 16 * o + n];
   }
   float lnw_tm[FT], lnb_tm[FT];
 #pragma unroll

@@ -38,6 +38,7 @@ namespace {
 struct SmallArgs {
   const void *XQ, *XK, *XV, *eta, *dout;
   const float *ln_w, *ln_b, *W1_init, *b1_init, *W2_init, *b2_init;
+  int NI;  // distinct initial states: chain c starts from state c % NI
   void* out;
   float *last[4], *ckpt[4], *memo[4];  // W1, b1, W2, b2 of one chain's [n] state sets (may be null)
   void *dXQ, *dXK, *dXV, *deta;
@@ -735,8 +736,9 @@ __global__ __launch_bounds__(64) void small_mlp_fwd_kernel(SmallArgs a) {
 
   Tile cW1[FT][HT], cW2[HT][FT];
   f4 b2T[FT];
-  load_mlp_state<FT, HT>(a.W1_init + chain * F * FF, a.b1_init + chain * FF, a.W2_init + chain * FF * F,
-                         a.b2_init + chain * F, cW1, cW2, sb1, b2T);
+  const size_t ic = chain % (size_t)a.NI;
+  load_mlp_state<FT, HT>(a.W1_init + ic * F * FF, a.b1_init + ic * FF, a.W2_init + ic * FF * F, a.b2_init + ic * F,
+                         cW1, cW2, sb1, b2T);
   f4 lw[FT], lb[FT];
   load_ln<FT>(a, h, lw, lb);
   float* states = a.saved + chain * a.per_chain + a.states;
@@ -1566,7 +1568,8 @@ __global__ __launch_bounds__(64) void small_lin_fwd_kernel(SmallArgs a) {
   const int h = (int)(chain % a.H), NC = a.NC;
   Tile cW[FT][FT];
   f4 bT[FT];
-  load_lin_state<FT>(a.W1_init + chain * F * F, a.b1_init + chain * F, cW, bT);
+  const size_t ic = chain % (size_t)a.NI;
+  load_lin_state<FT>(a.W1_init + ic * F * F, a.b1_init + ic * F, cW, bT);
   f4 lw[FT], lb[FT];
   load_ln<FT>(a, h, lw, lb);
   float* states = a.saved + chain * a.per_chain + a.states;
@@ -1906,6 +1909,7 @@ hipError_t launch_small_fwd(const GenFwdParams& q, int dtype, hipStream_t stream
   a.ln_w = q.ln_w;
   a.ln_b = q.ln_b;
   a.W1_init = q.W1_init;
+  a.NI = q.NI;
   a.b1_init = q.b1_init;
   a.W2_init = q.W2_init;
   a.b2_init = q.b2_init;

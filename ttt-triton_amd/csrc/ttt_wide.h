@@ -100,7 +100,7 @@ struct WideArgs {
   void *dXQ, *dXK, *dXV, *deta;
   float *dW1, *db1, *dW2, *db2, *dln_w, *dln_b;
   float* saved;
-  int H, NC, G, M, eta_rule;
+  int H, NC, G, M, NI, eta_rule;
   float eps;
 };
 

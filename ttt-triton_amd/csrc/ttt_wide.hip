@@ -53,6 +53,7 @@ hipError_t launch_wide_fwd(const GenFwdParams& q, int dtype, hipStream_t stream)
   a.ln_w = q.ln_w;
   a.ln_b = q.ln_b;
   a.W1_init = q.W1_init;
+  a.NI = q.NI;
   a.b1_init = q.b1_init;
   a.W2_init = q.W2_init;
   a.b2_init = q.b2_init;

@@ -59,6 +59,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
   const int NK = (NC + a.G - 1) / a.G, NS = (NC + a.M - 1) / a.M;
   float* const slot0 = a.saved + chain * NC * (size_t)Sl::FLOATS;
 
+  const size_t ic = chain % (size_t)a.NI;
   f4 w1[NSL][NT], w2[NSL][NT];
 #pragma unroll
   for (int sl = 0; sl < NSL; ++sl)
@@ -67,16 +68,16 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
       const int t = w + n * C::NW;
       if (C::ALLT || t < C::TW) {
         const WideTile<4> t1(t);
-        w1[sl][n] = ldf4(t1.template at<FF>(a.W1_init + chain * F * FF + sl * 64));
+        w1[sl][n] = ldf4(t1.template at<FF>(a.W1_init + ic * F * FF + sl * 64));
         if constexpr (MLP) {
           const WideTile<C::FT> t2(t);
-          w2[sl][n] = ldf4(t2.template at<F>(a.W2_init + (chain * FF + sl * 64) * F));
+          w2[sl][n] = ldf4(t2.template at<F>(a.W2_init + (ic * FF + sl * 64) * F));
         }
       }
     }
-  for (int i = tid; i < FF; i += C::NTH) b1s[i] = a.b1_init[chain * FF + i];
+  for (int i = tid; i < FF; i += C::NTH) b1s[i] = a.b1_init[ic * FF + i];
   if (MLP)
-    for (int i = tid; i < F; i += C::NTH) b2s[i] = a.b2_init[chain * F + i];
+    for (int i = tid; i < F; i += C::NTH) b2s[i] = a.b2_init[ic * F + i];
 
   // destination i of the state entering mini-batch s (s = NC: the final one):
   // the next slot, a checkpoint, the final state, a memo snapshot.  The

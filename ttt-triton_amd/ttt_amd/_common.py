@@ -29,6 +29,16 @@ def f32c(t: torch.Tensor) -> torch.Tensor:
     return as_act(t, torch.float32)
 
 
+def states(ts):
+    """(initial fast weights as the kernels read them, STATE_SHARED or 0): a batch
+    expanded from one state ([H,...] with batch stride 0, as the layer passes it)
+    is read in place, anything else as a contiguous fp32 [B,H,...]."""
+    if all(t.dtype == torch.float32 and t.stride() == (0, t.shape[2] * t.shape[3], t.shape[3], 1)
+           and ptr(t) % 16 == 0 for t in ts):
+        return ts, _lib.STATE_SHARED
+    return [f32c(t) for t in ts], 0
+
+
 def eta_operand(eta: torch.Tensor, rule: int, dt: torch.dtype):
     """(eta as the kernels read it, the rule code to pass).  A dense eta keeps
     its own dtype when that is fp32 under 16-bit activations (TTT_ETA_DENSE_F32,

@@ -28,6 +28,7 @@ ETA_LAYER = 1
 ETA_CAUSAL = 2
 ETA_DENSE_F32 = 3  # dense eta kept in fp32 under 16-bit activations (chosen from eta's dtype)
 FORM_SPLIT = 0x100  # or'ed into the eta rule: the state and the readout as two launches
+STATE_SHARED = 0x200  # (forward): initial states [H,...], one for every sequence
 ETA_RULES = {"dense": ETA_DENSE, "layer": ETA_LAYER, "causal": ETA_CAUSAL}
 
 # process-wide options (enum ttt_option)

@@ -14,7 +14,7 @@ import math
 import torch
 
 from . import _lib
-from ._common import as_act, check_device, dtype_code, eta_operand, f32c, grads_as, on_device, ptr, stream_of
+from ._common import as_act, check_device, dtype_code, eta_operand, f32c, grads_as, on_device, ptr, states, stream_of
 
 LN_EPS = 1e-8  # ops/ttt_utils.py:4,21
 
@@ -62,8 +62,8 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
     NK = math.ceil(NC / G)
     xq, xk, xv = (as_act(t, mp) for t in (XQ, XK, XV))
     et, krule = eta_operand(eta, rule, mp)
-    w1 = f32c(W1)
-    bb = f32c(b1)
+    (w1, bb), shared = states((W1, b1))
+    krule |= shared
     lw = f32c(ln_w)
     lb = f32c(ln_b)
     out = torch.empty((B, H, NC, K, F), device=dev, dtype=mp)

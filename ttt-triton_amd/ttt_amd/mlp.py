@@ -16,7 +16,8 @@ import os
 import torch
 
 from . import _lib
-from ._common import as_act, check_device, dtype_code, eta_operand, f32c, grads_as, on_device, ptr, stream_of
+from ._common import (as_act, check_device, dtype_code, eta_operand, f32c, grads_as, on_device, ptr, states,
+                      stream_of)
 
 LN_EPS = 1e-8  # ops/ttt_utils.py:4,21
 
@@ -77,7 +78,9 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     NK = math.ceil(NC / G)
     xq, xk, xv = (as_act(t, mp) for t in (XQ, XK, XV))
     et, krule = eta_operand(eta, rule, mp)
-    w1, bb1, w2, bb2, lw, lb = (f32c(t) for t in (W1, b1, W2, b2, ln_w, ln_b))
+    (w1, bb1, w2, bb2), shared = states((W1, b1, W2, b2))
+    krule |= shared
+    lw, lb = f32c(ln_w), f32c(ln_b)
     out = torch.empty((B, H, NC, K, F), device=dev, dtype=mp)
 
     def state(n, w1_only=False):
