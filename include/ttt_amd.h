@@ -297,6 +297,25 @@ int ttt_mlp_memo_combine_bwd(const void* XQ, const void* XU, const void* XQW, co
                              float* gates, size_t gates_bytes, void* dXK, void* dXU, void* dXQW,
                              void* stream);
 
+/* The pair of calls above with the readouts' rows kept in between:
+ * ttt_mlp_memo_combine_keep is ttt_mlp_memo_combine (the same output) that also
+ * writes, for every memo state and every token of a later segment, the centred
+ * row of its readout before the LayerNorm's scale and 1/sigma in fp32 (`rows`, >=
+ * ttt_mlp_memo_rows_bytes: F + 1 floats per pair); ttt_mlp_memo_combine_bwd_kept
+ * reads them instead of forming every readout again (the same gradients), and
+ * needs no memo state.  The rows grow with the square of the sequence (0 bytes for a single segment). */
+size_t ttt_mlp_memo_rows_bytes(int B, int H, int NC, int K, int F, int M);
+int ttt_mlp_memo_combine_keep(const void* XQ, const void* XK, const void* XU, const void* XQW,
+                              const float* W1_memo, const float* b1_memo, const float* W2_memo,
+                              const float* b2_memo, const float* ln_w, const float* ln_b,
+                              int B, int H, int NC, int K, int F, int FF, int M, int dtype, float eps,
+                              void* out, float* gates, size_t gates_bytes, float* rows, size_t rows_bytes,
+                              void* stream);
+int ttt_mlp_memo_combine_bwd_kept(const void* XQ, const void* XU, const void* XQW, const float* ln_w,
+                                  const float* ln_b, const void* dout, int B, int H, int NC, int K, int F, int M,
+                                  int dtype, float* gates, size_t gates_bytes, const float* rows, size_t rows_bytes,
+                                  void* dXK, void* dXU, void* dXQW, void* stream);
+
 /* ---- the producer and consumer around the inner loop (ttt_layer.py) ----
  * Shapes: B batch, L = NC*K tokens, H heads, F head dim (32 or 64), K a
  * multiple of 16 up to 64, D = H*F <= 1024.  Activations in `dtype`, everything else fp32. */

@@ -807,10 +807,10 @@ ttt::MlpMemoParams memo_params(const void* XQ, const void* XQW, const float* W1,
 }
 }  // namespace
 
-int ttt_mlp_memo_combine(const void* XQ, const void* XK, const void* XU, const void* XQW, const float* W1_memo,
+static int memo_combine_impl(const void* XQ, const void* XK, const void* XU, const void* XQW, const float* W1_memo,
                          const float* b1_memo, const float* W2_memo, const float* b2_memo, const float* ln_w,
                          const float* ln_b, int B, int H, int NC, int K, int F, int FF, int M, int dtype, float eps,
-                         void* out, float* gates, size_t gates_bytes, void* stream) {
+                         void* out, float* gates, size_t gates_bytes, float* rows, void* stream) {
   int st = check_memo(B, H, NC, K, F, FF, M, dtype, eps, gates_bytes, gates);
   if (st != TTT_OK) return st;
   const void* req[] = {XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, out};
@@ -821,9 +821,56 @@ int ttt_mlp_memo_combine(const void* XQ, const void* XK, const void* XU, const v
   p.XK = XK;
   p.XU = XU;
   p.out = out;
+  p.rows = rows;
   p.packed = memo_packed(gates, gates_bytes, B, H, NC, K, F, FF, M, dtype);
   if ((long long)B * H * p.nchunk > 0x7fffffffLL) return TTT_ERR_SHAPE;
   return hip_status(ttt::launch_mlp_memo(p, dtype, false, static_cast<hipStream_t>(stream)));
+}
+
+int ttt_mlp_memo_combine(const void* XQ, const void* XK, const void* XU, const void* XQW, const float* W1_memo,
+                         const float* b1_memo, const float* W2_memo, const float* b2_memo, const float* ln_w,
+                         const float* ln_b, int B, int H, int NC, int K, int F, int FF, int M, int dtype, float eps,
+                         void* out, float* gates, size_t gates_bytes, void* stream) {
+  return memo_combine_impl(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, B, H, NC, K, F, FF, M, dtype, eps, out,
+                           gates, gates_bytes, nullptr, stream);
+}
+
+size_t ttt_mlp_memo_rows_bytes(int B, int H, int NC, int K, int F, int M) {
+  if (ttt_mlp_memo_gates_bytes(B, H, NC, K, F, M) == 0) return 0;
+  return (size_t)B * H * ttt::mlp_memo_row_tiles(NC * (K / 16), M * (K / 16)) * 16 * (F + 1) * sizeof(float);
+}
+
+int ttt_mlp_memo_combine_keep(const void* XQ, const void* XK, const void* XU, const void* XQW, const float* W1_memo,
+                              const float* b1_memo, const float* W2_memo, const float* b2_memo, const float* ln_w,
+                              const float* ln_b, int B, int H, int NC, int K, int F, int FF, int M, int dtype,
+                              float eps, void* out, float* gates, size_t gates_bytes, float* rows, size_t rows_bytes,
+                              void* stream) {
+  REQUIRE_PTR(rows);
+  if (rows_bytes < ttt_mlp_memo_rows_bytes(B, H, NC, K, F, M)) return TTT_ERR_WORKSPACE;
+  return memo_combine_impl(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, B, H, NC, K, F, FF, M, dtype, eps, out,
+                           gates, gates_bytes, rows, stream);
+}
+
+int ttt_mlp_memo_combine_bwd_kept(const void* XQ, const void* XU, const void* XQW, const float* ln_w,
+                                  const float* ln_b, const void* dout, int B, int H, int NC, int K, int F, int M,
+                                  int dtype, float* gates, size_t gates_bytes, const float* rows, size_t rows_bytes,
+                                  void* dXK, void* dXU, void* dXQW, void* stream) {
+  int st = check_memo(B, H, NC, K, F, 64, M, dtype, 1e-6f, gates_bytes, gates);
+  if (st != TTT_OK) return st;
+  const void* req[] = {XQ, XU, XQW, ln_w, ln_b, dout, rows, dXK, dXU, dXQW};
+  for (const void* q : req) REQUIRE_PTR(q);
+  if (rows_bytes < ttt_mlp_memo_rows_bytes(B, H, NC, K, F, M)) return TTT_ERR_WORKSPACE;
+  if ((long long)B * H * NC * (K / 16) > 0x7fffffffLL) return TTT_ERR_SHAPE;
+  const int k = K / 16;  // 16-token tiles per mini-batch
+  ttt::MlpMemoParams p = memo_params(XQ, XQW, nullptr, nullptr, nullptr, nullptr, ln_w, ln_b, B, H, NC * k, F, 64,
+                                     M * k, 1e-6f, gates);
+  p.XU = XU;
+  p.dout = dout;
+  p.rows = const_cast<float*>(rows);
+  p.dXK = dXK;
+  p.dXU = dXU;
+  p.dXQW = dXQW;
+  return hip_status(ttt::launch_mlp_memo(p, dtype, true, static_cast<hipStream_t>(stream)));
 }
 
 int ttt_mlp_memo_combine_bwd(const void* XQ, const void* XU, const void* XQW, const float* W1_memo,

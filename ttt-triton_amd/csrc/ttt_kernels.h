@@ -102,12 +102,14 @@ struct MlpMemoParams {
   const float *W1, *b1, *W2, *b2, *ln_w, *ln_b;
   void *out, *dXK, *dXU, *dXQW;
   float* gates;
+  float* rows;  // the readouts' centred rows, then their 1/sigma, kept for the backward (mlp_memo_row_tiles), or null
   unsigned char* packed;  // bf16: [B*H][NS] LDS images of the memo states (mlp_memo_image_bytes each), or null
   int B, H, NC, F, FF, M, NS, nchunk;
   float eps;
 };
 size_t memo_gate_floats_per_chain(int NC, int K, int F, int M);
 size_t mlp_memo_image_bytes(int F, int FF);
+size_t mlp_memo_row_tiles(int NC, int M);  // [16 x F] tiles of kept rows per chain
 hipError_t launch_mlp_memo(const MlpMemoParams& p, int dtype, bool bwd, hipStream_t stream);
 int mlp_memo_chunk_tiles(int B, int H, int NC);  // mini-batches per combiner workgroup chunk
 

@@ -24,6 +24,12 @@
 //                         readout does), run the chunk's tiles of later
 //                         segments through R_j and accumulate gamma_j R_j (forward)
 //                         or dOut . R_j (backward: the gate gradients);
+//   memo_dgam_kernel      (backward, where the forward kept the readouts'
+//                         centred rows and 1/sigma) one wave per 16 tokens: the gate
+//                         gradients from the kept rows, instead of memo_combine_kernel
+//                         forming every readout again.  The combiner is bound by
+//                         its GELUs (433 us at B16 H12 T2048 F64 FF256 M8, bf16), the
+//                         kept rows are 755 MB written beside them and read back;
 //   memo_finish_kernel    (backward) one workgroup per 64 tokens: the softmax
 //                         backward, dXU = sum_j dsims_j summary_j and
 //                         dXQW = gamma_i dOut;
@@ -271,6 +277,11 @@ __global__ __launch_bounds__(256) void memo_pack_kernel(MlpMemoParams p) {
   for (int i = threadIdx.x; i < IMG / 16; i += 256) dst[i] = src[i];
 }
 
+// First kept tile of state j: the tiles of the segments after j, state by state.
+__host__ __device__ __forceinline__ size_t memo_row_tile0(int NC, int M, int j) {
+  return (size_t)j * NC - (size_t)M * j * (j + 1) / 2;
+}
+
 template <typename T, int FT, int HTT, bool BWD, bool PK, int NTW>
 __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoParams p) {
   constexpr int F = 16 * FT;
@@ -301,6 +312,9 @@ __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoPa
   const size_t xoff = (size_t)chain * NT * F;
   const T* __restrict__ XQ = static_cast<const T*>(p.XQ) + xoff;
   float* __restrict__ gb = p.gates + (size_t)chain * L.stride;
+  const size_t ctiles = memo_row_tile0(NC, M, NS - 1);  // kept tiles of a chain
+  float* const rows = !BWD && p.rows != nullptr ? p.rows + chain * ctiles * (16 * F) : nullptr;
+  float* const rstds = !BWD && p.rows != nullptr ? p.rows + p.B * p.H * ctiles * (16 * F) + chain * ctiles * 16 : nullptr;
 
 #pragma unroll 1
   for (int half = 0; half < 2; ++half) {
@@ -442,6 +456,13 @@ __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoPa
           const float gr = gjv[t] * rstd;
 #pragma unroll
           for (int c = 0; c < FT; ++c) oacc[t][c] += gr * acc[t][c].v;
+          if (rows != nullptr) {  // lane order, past the caches: read once, by the backward
+            const size_t i = memo_row_tile0(NC, M, jm) + (t0 + t - (jm + 1) * M);
+#pragma unroll
+            for (int c = 0; c < FT; ++c)
+              __builtin_nontemporal_store(acc[t][c].v, reinterpret_cast<f4*>(rows + i * (16 * F) + 256 * c) + l);
+            if (g == 0) __builtin_nontemporal_store(rstd, rstds + i * 16 + n);
+          }
         }
       }
       if constexpr (PK) {
@@ -471,6 +492,64 @@ __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoPa
       }
     }
   }  // half
+}
+
+// ------------------------------------------------------------------ backward: dgamma from the kept rows
+// dgamma_j = dOut . R_j = dOut . (XQ + ln_b) + rstd (dOut * ln_w) . V_j of one tile
+// per wave (V_j the centred rows, their products summed in the order that
+// memo_combine_kernel sums them), the tiles with the most states first.  Bound by the kept rows' bytes: four
+// states' loads are requested at a time.
+template <typename T, int FT> __global__ __launch_bounds__(256) void memo_dgam_kernel(MlpMemoParams p) {
+  constexpr int F = 16 * FT, K = 16, U = 4;
+  const int NC = p.NC, M = p.M, NS = p.NS, NT = NC * K, chains = p.B * p.H;
+  const long long idx = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (idx >= (long long)chains * (NC - M)) return;
+  const int chain = (int)(idx % chains), tile = NC - 1 - (int)(idx / chains), seg = tile / M;
+  const int h = chain % p.H;
+  const int l = lane_id(), g = l >> 4, n = l & 15;
+  const MemoGateLayout L(NC, K, F, NS);
+  float* __restrict__ dgam = p.gates + (size_t)chain * L.stride + L.dgam + (size_t)tile * K + n;
+  const size_t ctiles = memo_row_tile0(NC, M, NS - 1);
+  const float* __restrict__ rows = p.rows + chain * ctiles * (16 * F) + 4 * l;
+  const float* __restrict__ rstds = p.rows + chains * ctiles * (16 * F) + chain * ctiles * 16 + n;
+  const size_t e = (size_t)chain * NT * F + ((size_t)tile * K + n) * F + 4 * g;
+  f4 o[FT];
+  float base = 0.f;
+#pragma unroll
+  for (int c = 0; c < FT; ++c) {
+    const f4 dv = load4(static_cast<const T*>(p.dout) + e + 16 * c);
+    const f4 xq = load4(static_cast<const T*>(p.XQ) + e + 16 * c);
+    f4 xb;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int f = h * F + 16 * c + 4 * g + j;
+      xb[j] = xq[j] + p.ln_b[f];
+      o[c][j] = dv[j] * p.ln_w[f];
+    }
+    base += (dv[0] * xb[0] + dv[1] * xb[1]) + (dv[2] * xb[2] + dv[3] * xb[3]);
+  }
+  base = sum_col4(base);
+  for (int j0 = 0; j0 < seg; j0 += U) {
+    f4 v[U][FT];
+    float rs[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int j = min(j0 + u, seg - 1);
+      const size_t i = memo_row_tile0(NC, M, j) + (tile - (j + 1) * M);
+#pragma unroll
+      for (int c = 0; c < FT; ++c)
+        v[u][c] = __builtin_nontemporal_load(reinterpret_cast<const f4*>(rows + i * (16 * F) + 256 * c));
+      rs[u] = __builtin_nontemporal_load(rstds + i * 16);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float d = 0.f;
+#pragma unroll
+      for (int c = 0; c < FT; ++c) d += (o[c][0] * v[u][c][0] + o[c][1] * v[u][c][1]) + (o[c][2] * v[u][c][2] + o[c][3] * v[u][c][3]);
+      d = base + rs[u] * sum_col4(d);
+      if (g == 0 && j0 + u < seg) dgam[(size_t)(j0 + u) * NT] = d;
+    }
+  }
 }
 
 // ------------------------------------------------------------------ backward: softmax, dXU, dXQW
@@ -667,7 +746,14 @@ template <typename T, int FT, int HTT>
 static hipError_t launch_memo_t(const MlpMemoParams& p, bool bwd, hipStream_t stream) {
   const int nrow = (p.NC * 16 + kTokBlk - 1) / kTokBlk;  // workgroups per chain of the gate and finish kernels
   if (bwd) {
-    hipError_t e = launch_combine<T, FT, HTT, true>(p, stream);
+    hipError_t e = hipSuccess;
+    if (p.rows == nullptr) {
+      e = launch_combine<T, FT, HTT, true>(p, stream);
+    } else if (p.NC > p.M) {
+      const long long tiles = (long long)p.B * p.H * (p.NC - p.M);
+      hipLaunchKernelGGL((memo_dgam_kernel<T, FT>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, stream, p);
+      e = hipGetLastError();
+    }
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL((memo_finish_kernel<T, 16 * FT>), dim3(p.B * p.H * nrow), dim3(kMemoThreads), 0, stream, p);
     e = hipGetLastError();
@@ -723,6 +809,8 @@ int mlp_memo_chunk_tiles(int B, int H, int NC) {
   const long long pairs = (long long)B * H * (((NC + kMemoChunkTiles - 1) / kMemoChunkTiles + 1) / 2);
   return pairs < kComputeUnits ? kMemoWaves : kMemoChunkTiles;
 }
+
+size_t mlp_memo_row_tiles(int NC, int M) { return memo_row_tile0(NC, M, (NC + M - 1) / M - 1); }
 
 size_t mlp_memo_image_bytes(int F, int FF) {
   const int FT = F / 16;

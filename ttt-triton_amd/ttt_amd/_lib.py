@@ -70,6 +70,9 @@ SIGNATURES = {
     "ttt_mlp_memo_gates_bytes": (_S, [_I] * 6),
     "ttt_mlp_memo_workspace_bytes": (_S, [_I] * 8),
     "ttt_mlp_memo_combine": (_I, [_P] * 10 + [_I] * 8 + [_F] + [_P, _P, _S, _P]),
+    "ttt_mlp_memo_rows_bytes": (_S, [_I] * 6),
+    "ttt_mlp_memo_combine_keep": (_I, [_P] * 10 + [_I] * 8 + [_F] + [_P, _P, _S, _P, _S, _P]),
+    "ttt_mlp_memo_combine_bwd_kept": (_I, [_P] * 6 + [_I] * 7 + [_P, _S, _P, _S] + [_P] * 4),
     "ttt_mlp_memo_combine_bwd": (_I, [_P] * 10 + [_I] * 8 + [_F] + [_P, _S, _P, _P, _P, _P]),
 }
 

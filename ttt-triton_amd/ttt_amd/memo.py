@@ -55,13 +55,15 @@ def _check(XQ, XK, XU, XQW, W1, b1, W2, b2, ln_w, ln_b, M):
 
 
 def memo_combine_forward(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M: int,
-                         eps: float = READOUT_EPS, images: bool = True):
+                         eps: float = READOUT_EPS, images: bool = True, rows=None):
     """Run the combiner.  Returns (out [B,H,NC,K,F] in XQW.dtype, gates) where
     `gates` (uint8 device buffer) is what memo_combine_backward needs.  With
     `images` (bf16), the workspace also holds each memo state's LDS image,
     written once here and copied straight into LDS by this call and the
     backward: worth its one conversion pass when a backward follows; without
-    it every workgroup converts the states it stages (the same results)."""
+    it every workgroup converts the states it stages (the same results).  `rows`
+    (a flat fp32 tensor of memo_rows floats) receives the readouts' centred rows
+    and their 1/sigma, from which the backward forms the gate gradients."""
     B, H, NC, K, F, FF, M = _check(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M)
     dev = check_device(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b)
     mp = XQW.dtype
@@ -76,9 +78,12 @@ def memo_combine_forward(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln
     gates = torch.empty(nbytes, device=dev, dtype=torch.uint8)
     out = torch.empty((B, H, NC, K, F), device=dev, dtype=mp)
     with on_device(dev):
-        st = lib.ttt_mlp_memo_combine(ptr(xq), ptr(xk), ptr(xu), ptr(xqw), *(ptr(t) for t in ws), ptr(lw), ptr(lb),
-                                      B, H, NC, K, F, FF, M, code, float(eps), ptr(out), ptr(gates), gates.numel(),
-                                      stream_of(dev))
+        args = (ptr(xq), ptr(xk), ptr(xu), ptr(xqw), *(ptr(t) for t in ws), ptr(lw), ptr(lb), B, H, NC, K, F, FF, M,
+                code, float(eps), ptr(out), ptr(gates), gates.numel())
+        if rows is None:
+            st = lib.ttt_mlp_memo_combine(*args, stream_of(dev))
+        else:
+            st = lib.ttt_mlp_memo_combine_keep(*args, ptr(rows), rows.numel() * 4, stream_of(dev))
     _lib.check(st, "ttt_mlp_memo_combine")
     return out, gates
 
@@ -104,25 +109,63 @@ def memo_combine_backward(XQ, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w,
     return dxk, dxu, dxqw
 
 
+# The kept rows grow with the square of the sequence: past this, the backward
+# forms the readouts again.
+ROWS_MAX_BYTES = 1 << 30
+
+
+def memo_rows(B: int, H: int, NC: int, K: int, F: int, M: int) -> int:
+    """Floats of the readouts' rows that a training forward keeps, 0
+    where there are none or they pass ROWS_MAX_BYTES."""
+    n = _lib.load().ttt_mlp_memo_rows_bytes(B, H, NC, K, F, M)
+    return n // 4 if n <= ROWS_MAX_BYTES else 0
+
+
+def memo_combine_backward_kept(XQ, XU, XQW, ln_w, ln_b, M: int, gates, rows, dout):
+    """memo_combine_backward from the rows that the forward kept."""
+    B, H, NC, K, F = XQ.shape
+    dev = check_device(XQ, XU, XQW, ln_w, ln_b, gates, rows, dout)
+    mp = XQW.dtype
+    xq, xu, xqw, do = (as_act(t, mp) for t in (XQ, XU, XQW, dout))
+    lw, lb = f32c(ln_w), f32c(ln_b)
+    dxk, dxu, dxqw = (torch.empty((B, H, NC, K, F), device=dev, dtype=mp) for _ in range(3))
+    with on_device(dev):
+        st = _lib.load().ttt_mlp_memo_combine_bwd_kept(
+            ptr(xq), ptr(xu), ptr(xqw), ptr(lw), ptr(lb), ptr(do), B, H, NC, K, F, int(M), dtype_code(mp), ptr(gates),
+            gates.numel(), ptr(rows), rows.numel() * 4, ptr(dxk), ptr(dxu), ptr(dxqw), stream_of(dev))
+    _lib.check(st, "ttt_mlp_memo_combine_bwd_kept")
+    return dxk, dxu, dxqw
+
+
 class MemoCombineFunction(torch.autograd.Function):
     """apply(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M[, eps]) -> out.
     Differentiable wrt XK, XU and XQW (as the reference's loop is)."""
 
     @staticmethod
     def forward(ctx, XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M, eps=READOUT_EPS):
-        # the memo-state images pay off only when the backward runs too
+        # the memo-state images pay off only when the backward stages the states too
         training = any(ctx.needs_input_grad[1:4])
+        n = memo_rows(*XQ.shape, int(M)) if training and XQ.dim() == 5 and int(M) > 0 else 0
+        rows = torch.empty(n, device=XQ.device, dtype=torch.float32) if n else None
         out, gates = memo_combine_forward(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M, eps,
-                                          images=training)
-        ctx.save_for_backward(XQ, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, gates)
+                                          images=training and not n, rows=rows)
+        if n:
+            ctx.save_for_backward(XQ, XU, XQW, ln_w, ln_b, gates, rows)
+        else:
+            ctx.save_for_backward(XQ, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, gates)
         ctx.M, ctx.eps = int(M), eps
         ctx.dtypes = (XK.dtype, XU.dtype, XQW.dtype)
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        XQ, XU, XQW, W1, b1, W2, b2, lw, lb, gates = ctx.saved_tensors
-        dxk, dxu, dxqw = memo_combine_backward(XQ, XU, XQW, W1, b1, W2, b2, lw, lb, ctx.M, gates, dout, ctx.eps)
+        saved = ctx.saved_tensors
+        if len(saved) == 7:
+            XQ, XU, XQW, lw, lb, gates, rows = saved
+            dxk, dxu, dxqw = memo_combine_backward_kept(XQ, XU, XQW, lw, lb, ctx.M, gates, rows, dout)
+        else:
+            XQ, XU, XQW, W1, b1, W2, b2, lw, lb, gates = saved
+            dxk, dxu, dxqw = memo_combine_backward(XQ, XU, XQW, W1, b1, W2, b2, lw, lb, ctx.M, gates, dout, ctx.eps)
         return (None,) + grads_as((dxk, dxu, dxqw), ctx.dtypes) + (None,) * 8
 
 
