@@ -119,7 +119,8 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
 size_t ttt_linear_saved_bytes(int B, int H, int NC, int K, int F);
 
 /* Bytes of the saved buffer of the split form (TTT_FORM_SPLIT; FF = 0: the
- * Linear loop): K = 16 with F = 64 (MLP: FF = 64, or F = 32 with FF = 128); 0 for any other shape. */
+ * Linear loop): K = 16 with F = 64 (MLP: FF = 64 or 256, or F = 32 with FF =
+ * 128); 0 for any other shape. */
 size_t ttt_split_saved_bytes(int B, int H, int NC, int K, int F, int FF);
 
 /* TTT-Linear backward: gradients of sum(out * dout) wrt every input, the

@@ -17,7 +17,7 @@ F32 = torch.float32
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["causal", "layer"])
-@pytest.mark.parametrize("F_,FF", [(64, 64), (32, 128)])
+@pytest.mark.parametrize("F_,FF", [(64, 64), (64, 256), (32, 128)])
 def test_mlp(F_, FF, kind):
     dt = F32
     from ttt_amd.mlp import mlp_backward, mlp_forward
@@ -59,7 +59,7 @@ def test_linear(kind):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("rule", ["dense", "layer", "causal"])
-@pytest.mark.parametrize("F_,FF", [(64, 0), (64, 64), (32, 128)])
+@pytest.mark.parametrize("F_,FF", [(64, 0), (64, 64), (64, 256), (32, 128)])
 def test_matches_the_specialised_kernels(F_, FF, rule):
     """Through the autograd Functions on both sides of the rule's chain count,
     a non-contiguous query among the inputs: a batch just past it takes the
@@ -68,7 +68,7 @@ def test_matches_the_specialised_kernels(F_, FF, rule):
     from ttt_amd.linear import TTTLinearFunction
     from ttt_amd.mlp import TTTMLPFunction
     H, NC, n = 1, 3, 5
-    B = (64 if FF else 128) + 1
+    B = (32 if FF == 256 else 64 if FF else 128) + 1
     d = _inputs(B, H, NC, 16, F_, FF, F32, "causal", 3 * F_ + FF)
     keys, fn = (MLP_KEYS, TTTMLPFunction) if FF else (LIN_KEYS, TTTLinearFunction)
     lr = torch.rand(B, H, NC, 16, generator=torch.Generator().manual_seed(F_)) / F_
@@ -101,9 +101,10 @@ def test_rule():
     assert _lib.split_form(x(2, 4, 16, 16, 64), 0) and _lib.split_form(x(2, 4, 16, 16, 32), 128)
     assert _lib.split_form(x(1, 64, 8, 16, 64), 64) and not _lib.split_form(x(1, 65, 8, 16, 64), 64)
     assert _lib.split_form(x(2, 64, 8, 16, 64), 0) and not _lib.split_form(x(2, 65, 8, 16, 64), 0)
+    assert _lib.split_form(x(1, 32, 8, 16, 64), 256)
     for dt in (torch.bfloat16, torch.float16):
         assert not _lib.split_form(x(2, 4, 16, 16, 64, dt=dt), 0)
-    for shape, FF in (((2, 4, 16, 32, 64), 0), ((2, 4, 16, 16, 32), 0), ((2, 4, 16, 16, 64), 256),
+    for shape, FF in (((2, 4, 16, 32, 64), 0), ((2, 4, 16, 16, 32), 0), ((1, 33, 16, 16, 64), 256),
                       ((2, 4, 16, 16, 64), 128), ((0, 4, 16, 16, 64), 0), ((2, 4, 16, 64), 0)):
         assert not _lib.split_form(x(*shape), FF), (shape, FF)
     lib = _lib.load()

@@ -9,8 +9,7 @@ namespace {
 template <int KT, typename Fn> size_t wide_visit_kt(int F, int FF, bool mlp, Fn f) {
   if (!mlp) return F == 64 ? f(WideShape<KT, 4, 1, false>{}) : 0;
   if (F == 64 && FF == 64) return f(WideShape<KT, 4, 1, true>{});
-  if constexpr (KT > 1)
-    if (F == 64 && FF == 256) return f(WideShape<KT, 4, 4, true>{});
+  if (F == 64 && FF == 256) return f(WideShape<KT, 4, 4, true>{});
   if (F == 32 && FF == 128) return f(WideShape<KT, 2, 2, true>{});
   return 0;
 }

@@ -1,19 +1,26 @@
 // Launchers of the ttt_wide.h kernels for one activation type.
 #pragma once
 
+#include "ttt_wave16.h"
 #include "ttt_wide_bwd.h"
 
 namespace ttt {
 namespace {
 
 template <typename T, class C> hipError_t wide_fwd(const WideArgs& a, int chains, hipStream_t stream) {
-  hipLaunchKernelGGL((wide_fwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
+  if constexpr (std::is_same_v<C, W16>)
+    hipLaunchKernelGGL(wave16_fwd_state_kernel, dim3(chains), dim3(kW16Threads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((wide_fwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
   hipLaunchKernelGGL((wide_fwd_readout_kernel<T, C>), dim3(chains * a.NC), dim3(C::NTH), 0, stream, a);
   return hipGetLastError();
 }
 template <typename T, class C> hipError_t wide_bwd(const WideArgs& a, int chains, hipStream_t stream) {
   hipLaunchKernelGGL((wide_bwd_readout_kernel<T, C>), dim3(chains * a.NC), dim3(C::NTH), 0, stream, a);
-  hipLaunchKernelGGL((wide_bwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
+  if constexpr (std::is_same_v<C, W16>)
+    hipLaunchKernelGGL(wave16_bwd_state_kernel, dim3(chains), dim3(kW16Threads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((wide_bwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -24,8 +31,7 @@ template <typename T, int KT> hipError_t wide_kt(const WideArgs& a, int F, int F
              : wide_fwd<T, WideShape<KT, FT, NSL, MLP>>(a, chains, stream)
   if (!mlp) TTT_WIDE(4, 1, false);
   if (F == 64 && FF == 64) TTT_WIDE(4, 1, true);
-  if constexpr (KT > 1)
-    if (F == 64 && FF == 256) TTT_WIDE(4, 4, true);
+  if (F == 64 && FF == 256) TTT_WIDE(4, 4, true);
   if (F == 32 && FF == 128) TTT_WIDE(2, 2, true);
 #undef TTT_WIDE
   return hipErrorInvalidValue;

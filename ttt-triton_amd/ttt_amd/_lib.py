@@ -135,10 +135,11 @@ def split_form(XQ, FF: int) -> bool:
     Kernel times specialised / split, 32 mini-batches, forward + backward at
     8, 64, 128 (96) chains: Linear 342/195, 348/239, 353/338 us (192 chains:
     359/415); MLP F = FF = 64 547/378, 559/474, (579/581); F = 32, FF = 128
-    734/479, 741/584, (758/705).  In 16 bits the specialised kernels' shorter
-    products win at every count (Linear 120/198 at 8 chains), and at F = 64,
-    FF = 256 in fp32 (1239/1505)."""
-    if XQ.dim() != 5 or XQ.dtype != torch.float32 or XQ.shape[0] * XQ.shape[1] > (64 if FF else 128):
+    734/479, 741/584, (758/705); F = 64, FF = 256 1241/946 at 8, 1253/1114 at 32,
+    1275/1342 at 64.  In 16 bits the specialised kernels' shorter products win at
+    every count (Linear 120/198 at 8 chains)."""
+    most = 32 if FF == 256 else 64 if FF else 128
+    if XQ.dim() != 5 or XQ.dtype != torch.float32 or XQ.shape[0] * XQ.shape[1] > most:
         return False
     return 0 < load().ttt_split_saved_bytes(*XQ.shape, FF) <= SPLIT_MAX_BYTES
 

@@ -65,7 +65,7 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     state-update operands and activations (a flat uint8 buffer of
     ttt_mlp_saved_bytes).  The backward reads only W1's checkpoints: with
     ckpt_w1_only the other three are neither allocated nor written (None).
-    With `split` (fp32, K = 16; F = FF = 64, or F = 32 with FF = 128)
+    With `split` (fp32, K = 16; F = 64 with FF 64 or 256, F = 32 with FF = 128)
     the state and the readout run as two launches (TTT_FORM_SPLIT): the saved
     buffer is then ttt_split_saved_bytes long, always allocated, and all that a
     split backward needs."""
