@@ -33,18 +33,6 @@ constexpr int kRowLd = 68;  // [16][64] rows in LDS: 16-byte row reads and 4-byt
 constexpr int kColLd = 20;  // [64][16] columns in LDS
 
 __device__ __forceinline__ Frag<float> fr(f4 v) { return Frag<float>{v}; }
-// The lane index, opaque once per mini-batch: what follows from it (some forty
-// addresses) is then formed where it is used instead of being kept, in registers
-// that 16 waves do not have, through the loop.
-__device__ __forceinline__ int pinned(int l) {
-  asm volatile("" : "+v"(l));
-  return l & 63;  // (its range known again: 32-bit address offsets)
-}
-// The same for a slot's index: its addresses stay a scalar base and a lane offset.
-__device__ __forceinline__ size_t pinned_index(size_t m) {
-  asm volatile("" : "+s"(m));
-  return m;
-}
 // 16-byte row read of an operand: free index r = lane % 16, contraction 4g + j
 template <int LD> __device__ __forceinline__ Frag<float> row_frag(const float* m, int l) {
   return fr(ldf4(m + (l & 15) * LD + 4 * (l >> 4)));

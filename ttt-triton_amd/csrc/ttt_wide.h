@@ -18,7 +18,7 @@
 // (the Linear loop has one layer: G, no P; the same four launches.)
 //
 // Measured at B32 H4, 8 mini-batches of 64 tokens, F = FF = 64, bf16, forward +
-// backward: 511 us (MLP; state 78 + 247, readouts 54 + 132), where the
+// backward: 431 us (MLP; state 76 + 172, readouts 53 + 130), where the
 // general-shape kernels (one workgroup per chain for everything, every matrix
 // through global scratch) take 6,780; the Linear loop 201 us against 3,090.
 // The shapes taken are those that a layer (FF = F) or the 4x MLP builds of
@@ -52,12 +52,21 @@ template <int KT_, int FT_, int NSL_, bool MLP_> struct WideShape {
   static constexpr int NT = (TW + NW - 1) / NW;  // of those, per wave
   // whether every wave has a tile in each pass over them (no branch then)
   static constexpr bool ALLT = TW % NW == 0, ALLF = FT == 4, ALLK = KT == 4;
+  // the state launches of 16 waves, MLP: addresses out of the registers (see pinned:
+  // backward at K = F = FF = 64, B32 H4, 8 mini-batches 247 -> 172 us)
+  static constexpr bool PIN = KT == 4 && MLP;
   // LDS rows are padded by 4 floats: row-major float4 reads (16 rows x 4 lane
   // groups) and column reads (4 rows x 16 lanes) both touch 64 distinct banks
   static constexpr int LS = S + 4, LF = F + 4, LK = K + 4;
   static constexpr int SLOT = 64 * LS;     // one LDS matrix of up to 64 x 64
   static constexpr int KSLOT = K * LS;     // one of K rows
   static_assert(MLP || (FT == 4 && NSL == 1), "the Linear loop: 64 features, one slice");
+};
+
+// the readout launches, which have registers to spare and no loop: not pinned
+template <class C> struct WideFree {
+  static constexpr int KT = C::KT;
+  static constexpr bool PIN = false;
 };
 
 // floats of one (chain, mini-batch) slot of `saved`
@@ -104,6 +113,19 @@ struct WideArgs {
   float eps;
 };
 
+// The lane index, opaque once per use: what follows from it (some forty addresses)
+// is then formed where it is used instead of being kept through a loop in registers
+// that 16 waves do not have.
+__device__ __forceinline__ int pinned(int l) {
+  asm volatile("" : "+v"(l));
+  return l & 63;  // (its range known again: 32-bit address offsets)
+}
+// The same for a slot's index: its addresses stay a scalar base and a lane offset.
+__device__ __forceinline__ size_t pinned_index(size_t m) {
+  asm volatile("" : "+s"(m));
+  return m;
+}
+
 // ---------------------------------------------------------------- products
 // c + op(A) op(B) for one 16 x 16 output tile, contraction KD (a multiple of
 // 16): A and B point at the tile's first row (column) of op(A) (op(B)) in
@@ -120,7 +142,7 @@ struct WideArgs {
 constexpr int kSchedKeepLdsReads = 0x2 | 0x4 | 0x70 | 0x200;
 template <class C, int KD, bool TA, bool TB, int LA, int LB, bool CS = false>
 __device__ __forceinline__ f4 wmm(f4 c, const float* A, const float* B, float* cs = nullptr) {
-  const int l = lane_id(), g = l >> 4, r = l & 15;
+  const int l = C::PIN ? pinned(lane_id()) : lane_id(), g = l >> 4, r = l & 15;
   const float* ap = TA ? A + 4 * g * LA + r : A + r * LA + 4 * g;
   const float* bp = TB ? B + r * LB + 4 * g : B + 4 * g * LB + r;
   Frag<float> a[KD / 16], b[KD / 16];
@@ -159,15 +181,15 @@ template <class C> __device__ __forceinline__ int wide_wave() {
 
 // the 16 x 16 tile grid of an R x Cc-tile product over the waves: tile w
 template <int CT> struct WideTile {
-  int it, jt;
-  __device__ __forceinline__ explicit WideTile(int t) : it(t / CT), jt(t % CT) {}
-  __device__ __forceinline__ int row() const { return 16 * it + (lane_id() & 15); }
-  __device__ __forceinline__ int col() const { return 16 * jt + 4 * (lane_id() >> 4); }
+  int it, jt, l;
+  __device__ __forceinline__ explicit WideTile(int t, int lane = lane_id()) : it(t / CT), jt(t % CT), l(lane) {}
+  __device__ __forceinline__ int row() const { return 16 * it + (l & 15); }
+  __device__ __forceinline__ int col() const { return 16 * jt + 4 * (l >> 4); }
   // this lane's four columns in a matrix of row width LD: the tile's part of the
   // address is uniform over the wave, the lane's an unsigned offset (global
   // accesses then take a scalar base and one 32-bit register per row width)
   template <int LD, class P> __device__ __forceinline__ P* at(P* base) const {
-    return base + (16 * it * LD + 16 * jt) + ((unsigned)(lane_id() & 15) * LD + 4u * (lane_id() >> 4));
+    return base + (16 * it * LD + 16 * jt) + ((unsigned)(l & 15) * LD + 4u * (unsigned)(l >> 4));
   }
 };
 

@@ -67,12 +67,12 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
   f4 dxq = zero;              // of its K x F tile
   float* const DA = C::MLP ? ro.G2 : ro.W2;  // d(X2b X2^T), then d(XQ XK^T)
   if (C::ALLK || ro.has_k) {
-    const f4 dc = wmm<C, F, false, true, LF, LF>(zero, ro.Z + 16 * tk.it * LF, ro.G2 + 16 * tk.jt * LF);  // -dC
+    const f4 dc = wmm<WideFree<C>, F, false, true, LF, LF>(zero, ro.Z + 16 * tk.it * LF, ro.G2 + 16 * tk.jt * LF);  // -dC
     deta = -(dc * ((C::MLP ? ro.a2 : ro.a1) + 1.0f));
     da = -(dc * ro.eta);
   }
   if (C::ALLF || ro.has_f) {  // -C^T dZ2b
-    const f4 t = wmm<C, K, true, false, LK, LF>(zero, ro.C1 + 16 * tf.it, ro.Z + 16 * tf.jt);
+    const f4 t = wmm<WideFree<C>, K, true, false, LK, LF>(zero, ro.C1 + 16 * tf.it, ro.Z + 16 * tf.jt);
     stf4(tf.template at<F>(slot + Sl::HG2), t);
   }
   float cs;
@@ -91,10 +91,10 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       stf4(ts.template at<LS>(ro.X2), x2);
       stf4(ts.template at<LS>(ro.XB), ro.xb[sl]);
       __syncthreads();
-      f4 dz = wmm<C, F, false, true, LF, LF>(zero, ro.Z + 16 * ts.it * LF, ro.W2 + 16 * ts.jt * LF);
-      dz = wmm<C, K, false, false, LK, LS>(dz, DA + 16 * ts.it * LK, ro.X2 + 16 * ts.jt);
+      f4 dz = wmm<WideFree<C>, F, false, true, LF, LF>(zero, ro.Z + 16 * ts.it * LF, ro.W2 + 16 * ts.jt * LF);
+      dz = wmm<WideFree<C>, K, false, false, LK, LS>(dz, DA + 16 * ts.it * LK, ro.X2 + 16 * ts.jt);
       dz *= ro.db[sl];
-      stf4(ts.template at<FF>(slot + Sl::HX2 + sl * 64), wmm<C, K, true, false, LK, LS>(zero, DA + 16 * ts.it, ro.XB + 16 * ts.jt));
+      stf4(ts.template at<FF>(slot + Sl::HX2 + sl * 64), wmm<WideFree<C>, K, true, false, LK, LS>(zero, DA + 16 * ts.it, ro.XB + 16 * ts.jt));
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
@@ -102,10 +102,10 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
           const WideTile<C::FT> t2(t);
           f4 dw;
           if (sl == 0 && t2.it == 0) {
-            dw = wmm<C, K, true, false, LS, LF, true>(zero, ro.XB, ro.Z + 16 * t2.jt, &cs);
+            dw = wmm<WideFree<C>, K, true, false, LS, LF, true>(zero, ro.XB, ro.Z + 16 * t2.jt, &cs);
             if (lane < 16) slot[Sl::HST + Sl::B2 + 16 * t2.jt + lane] = cs;
           } else {
-            dw = wmm<C, K, true, false, LS, LF>(zero, ro.XB + 16 * t2.it, ro.Z + 16 * t2.jt);
+            dw = wmm<WideFree<C>, K, true, false, LS, LF>(zero, ro.XB + 16 * t2.it, ro.Z + 16 * t2.jt);
           }
           stf4(t2.template at<F>(slot + Sl::HST + Sl::W2 + sl * 64 * F), dw);
         }
@@ -115,9 +115,9 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       stf4(ts.template at<LS>(ro.X2), g1);
       ro.stage_w1(sl);
       __syncthreads();
-      if (C::ALLF || ro.has_f) dxq = wmm<C, C::S, false, true, LS, LS>(dxq, ro.XB + 16 * tf.it * LS, ro.W1 + 16 * tf.jt * LS);
-      if (C::ALLK || ro.has_k) dc1 = wmm<C, C::S, false, true, LS, LS>(dc1, ro.XB + 16 * tk.it * LS, ro.X2 + 16 * tk.jt * LS);
-      stf4(ts.template at<FF>(slot + Sl::HG1 + sl * 64), wmm<C, K, true, false, LK, LS>(zero, ro.C1 + 16 * ts.it, ro.XB + 16 * ts.jt));
+      if (C::ALLF || ro.has_f) dxq = wmm<WideFree<C>, C::S, false, true, LS, LS>(dxq, ro.XB + 16 * tf.it * LS, ro.W1 + 16 * tf.jt * LS);
+      if (C::ALLK || ro.has_k) dc1 = wmm<WideFree<C>, C::S, false, true, LS, LS>(dc1, ro.XB + 16 * tk.it * LS, ro.X2 + 16 * tk.jt * LS);
+      stf4(ts.template at<FF>(slot + Sl::HG1 + sl * 64), wmm<WideFree<C>, K, true, false, LK, LS>(zero, ro.C1 + 16 * ts.it, ro.XB + 16 * ts.jt));
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
@@ -125,10 +125,10 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
           const WideTile<4> t1(t);
           f4 dw;
           if (t1.it == 0) {
-            dw = wmm<C, K, true, false, LF, LS, true>(zero, ro.XQ, ro.XB + 16 * t1.jt, &cs);
+            dw = wmm<WideFree<C>, K, true, false, LF, LS, true>(zero, ro.XQ, ro.XB + 16 * t1.jt, &cs);
             if (lane < 16) slot[Sl::HST + Sl::B1 + sl * 64 + 16 * t1.jt + lane] = cs;
           } else {
-            dw = wmm<C, K, true, false, LF, LS>(zero, ro.XQ + 16 * t1.it, ro.XB + 16 * t1.jt);
+            dw = wmm<WideFree<C>, K, true, false, LF, LS>(zero, ro.XQ + 16 * t1.it, ro.XB + 16 * t1.jt);
           }
           stf4(t1.template at<FF>(slot + Sl::HST + Sl::W1 + sl * 64), dw);
         }
@@ -141,7 +141,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       stf4(tk.template at<LK>(DA), da);
     }
   } else {
-    dxq = wmm<C, F, false, true, LF, LS>(zero, ro.Z + 16 * tf.it * LF, ro.W1 + 16 * tf.jt * LS);
+    dxq = wmm<WideFree<C>, F, false, true, LF, LS>(zero, ro.Z + 16 * tf.it * LF, ro.W1 + 16 * tf.jt * LS);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const int t = w + n * C::NW;
@@ -149,10 +149,10 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
         const WideTile<4> t1(t);
         f4 dw;
         if (t1.it == 0) {
-          dw = wmm<C, K, true, false, LF, LF, true>(zero, ro.XQ, ro.Z + 16 * t1.jt, &cs);
+          dw = wmm<WideFree<C>, K, true, false, LF, LF, true>(zero, ro.XQ, ro.Z + 16 * t1.jt, &cs);
           if (lane < 16) slot[Sl::HST + Sl::B1 + 16 * t1.jt + lane] = cs;
         } else {
-          dw = wmm<C, K, true, false, LF, LF>(zero, ro.XQ + 16 * t1.it, ro.Z + 16 * t1.jt);
+          dw = wmm<WideFree<C>, K, true, false, LF, LF>(zero, ro.XQ + 16 * t1.it, ro.Z + 16 * t1.jt);
         }
         stf4(t1.template at<F>(slot + Sl::HST + Sl::W1), dw);
       }
@@ -180,9 +180,9 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
   }
   __syncthreads();
   if (C::ALLF || ro.has_f) {
-    dxq = wmm<C, K, false, false, LK, LF>(dxq, DA + 16 * tf.it * LK, ro.XK + 16 * tf.jt);
+    dxq = wmm<WideFree<C>, K, false, false, LK, LF>(dxq, DA + 16 * tf.it * LK, ro.XK + 16 * tf.jt);
     st4(tf.template at<F>(static_cast<T*>(a.dXQ) + m * K * F), dxq + frag_to_f4(ldraw4(tf.template at<F>(DO))));
-    stf4(tf.template at<F>(slot + Sl::HXK), wmm<C, K, true, false, LK, LF>(zero, DA + 16 * tf.it, ro.XQ + 16 * tf.jt));
+    stf4(tf.template at<F>(slot + Sl::HXK), wmm<WideFree<C>, K, true, false, LK, LF>(zero, DA + 16 * tf.it, ro.XQ + 16 * tf.jt));
   }
   if (lr_rule && tid < K) {
     float t = 0.f;
@@ -251,9 +251,16 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
     rp = ldf4(ts.template at<FF>(slot + Sl::P));
   }
 
+  const int lane0 = lane;
   for (int s = NC - 1; s >= 0; --s) {
     m = chain * NC + s;
-    slot = slot0 + (size_t)s * Sl::FLOATS;
+    if constexpr (C::PIN) m = pinned_index(m);
+    slot = a.saved + m * Sl::FLOATS;
+    const int lane = C::PIN ? pinned(lane0) : lane0, tid = 64 * w + lane;
+    const int prow = tid >> 4, pcol = (tid & 15) * V;
+    const unsigned po = (unsigned)(prow * F + pcol);
+    const WideTile<4> ts(w, lane);
+    const WideTile<C::FT> tf(w, lane);
     const vt rxv = ldact<T, V>(XV + m * K * F + po);
     const vf zh = ldv<V>(slot + Sl::ZH + po);
     const float sd = (slot + Sl::SIG)[(unsigned)prow];
@@ -272,7 +279,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
         if (C::ALLT || t < C::TW) {
-          const WideTile<4> t1(t);
+          const WideTile<4> t1(t, lane);
           stf4(t1.template at<LS>(G1s), ldf4(t1.template at<FF>(slot + Sl::W1 + sl * 64)));
         }
       }
@@ -282,7 +289,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
         if (C::ALLT || t < C::TW) {
-          const WideTile<C::FT> t2t(t);
+          const WideTile<C::FT> t2t(t, lane);
           stf4(t2t.template at<LF>(W2s), ldf4(t2t.template at<F>(slot + Sl::W2 + sl * 64 * F)));
         }
       }
@@ -307,8 +314,8 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
         for (int n = 0; n < NT; ++n) {
           const int t = w + n * C::NW;
           if (C::ALLT || t < C::TW) {
-            const WideTile<4> t1(t);
-            const WideTile<C::FT> t2t(t);
+            const WideTile<4> t1(t, lane);
+            const WideTile<C::FT> t2t(t, lane);
             stf4(t1.template at<LS>(DW1s), dw1[sl][n]);
             stf4(t2t.template at<LF>(DW2s), dw2[sl][n]);
           }
@@ -339,7 +346,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
         for (int n = 0; n < NT; ++n) {
           const int tt = w + n * C::NW;
           if (C::ALLT || tt < C::TW) {
-            const WideTile<C::FT> t2t(tt);
+            const WideTile<C::FT> t2t(tt, lane);
             dw2[sl][n] = wmm<C, K, true, false, LS, LF>(dw2[sl][n], DW1s + 16 * t2t.it, G2s + 16 * t2t.jt);
           }
         }
@@ -350,7 +357,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
         if (C::ALLT || t < C::TW) {
-          const WideTile<4> t1(t);
+          const WideTile<4> t1(t, lane);
           stf4(t1.template at<LS>(DW1s), dw1[0][n]);
         }
       }
@@ -445,7 +452,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
         for (int n = 0; n < NT; ++n) {
           const int t = w + n * C::NW;
           if (C::ALLT || t < C::TW) {
-            const WideTile<C::FT> t2t(t);
+            const WideTile<C::FT> t2t(t, lane);
             const f4 hw = ldf4(t2t.template at<F>(slot + Sl::HST + Sl::W2 + sl * 64 * F));
             if (sl == 0 && t2t.it == 0) {
               dw2[sl][n] = wmm<C, K, true, false, LS, LF, true>(dw2[sl][n], X2s, DGs + 16 * t2t.jt, &cs);
@@ -462,7 +469,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
         for (int n = 0; n < NT; ++n) {
           const int t = w + n * C::NW;
           if (C::ALLT || t < C::TW) {
-            const WideTile<4> t1(t);
+            const WideTile<4> t1(t, lane);
             const f4 hw = ldf4(t1.template at<FF>(slot + Sl::HST + Sl::W1 + sl * 64));
             if (t1.it == 0) {
               dw1[sl][n] = wmm<C, K, true, false, LF, LS, true>(dw1[sl][n], XKs, DW1s + 16 * t1.jt, &cs);
@@ -482,7 +489,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
         if (C::ALLT || t < C::TW) {
-          const WideTile<4> t1(t);
+          const WideTile<4> t1(t, lane);
           const f4 hw = ldf4(t1.template at<F>(slot + Sl::HST + Sl::W1));
           if (t1.it == 0) {
             dw1[0][n] = wmm<C, K, true, false, LF, LF, true>(dw1[0][n], XKs, DGs + 16 * t1.jt, &cs);

@@ -429,7 +429,7 @@ template <typename T, class C> struct WideReadout {
     __syncthreads();
     const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
     if (C::ALLK || has_k) {
-      a1 = wmm<C, F, false, true, LF, LF>(zero, XQ + 16 * tk.it * LF, XK + 16 * tk.jt * LF);
+      a1 = wmm<WideFree<C>, F, false, true, LF, LF>(zero, XQ + 16 * tk.it * LF, XK + 16 * tk.jt * LF);
       stf4(tk.template at<LK>(C1), -(eta * (a1 + 1.0f)));
     }
     f4 z = zero;
@@ -438,9 +438,9 @@ template <typename T, class C> struct WideReadout {
 #pragma unroll
       for (int sl = 0; sl < NSL; ++sl) {
         f4 zb = ldf4(slot + Sl::B1 + sl * 64 + ts.col());
-        zb = wmm<C, F, false, false, LF, LS>(zb, XQ + 16 * ts.it * LF, W1 + 16 * ts.jt);
+        zb = wmm<WideFree<C>, F, false, false, LF, LS>(zb, XQ + 16 * ts.it * LF, W1 + 16 * ts.jt);
         if (sl == 0) __syncthreads();  // C1
-        zb = wmm<C, K, false, false, LK, LS>(zb, C1 + 16 * ts.it * LK, Z + 16 * ts.jt);
+        zb = wmm<WideFree<C>, K, false, false, LK, LS>(zb, C1 + 16 * ts.it * LK, Z + 16 * ts.jt);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float y, dy;
@@ -450,8 +450,8 @@ template <typename T, class C> struct WideReadout {
         }
         stf4(ts.template at<LS>(XB), xb[sl]);
         __syncthreads();
-        if (C::ALLK || has_k) a2 = wmm<C, C::S, false, true, LS, LS>(a2, XB + 16 * tk.it * LS, X2 + 16 * tk.jt * LS);
-        if (C::ALLF || has_f) z = wmm<C, C::S, false, false, LS, LF>(z, XB + 16 * tf.it * LS, W2 + 16 * tf.jt);
+        if (C::ALLK || has_k) a2 = wmm<WideFree<C>, C::S, false, true, LS, LS>(a2, XB + 16 * tk.it * LS, X2 + 16 * tk.jt * LS);
+        if (C::ALLF || has_f) z = wmm<WideFree<C>, C::S, false, false, LS, LF>(z, XB + 16 * tf.it * LS, W2 + 16 * tf.jt);
         if (sl + 1 < NSL) {
           __syncthreads();
           stage_w1(sl + 1);
@@ -463,13 +463,13 @@ template <typename T, class C> struct WideReadout {
       if (C::ALLK || has_k) stf4(tk.template at<LK>(C1), -(eta * (a2 + 1.0f)));
       __syncthreads();
       if (C::ALLF || has_f) {
-        z = wmm<C, K, false, false, LK, LF>(z, C1 + 16 * tf.it * LK, G2 + 16 * tf.jt);
+        z = wmm<WideFree<C>, K, false, false, LK, LF>(z, C1 + 16 * tf.it * LK, G2 + 16 * tf.jt);
         stf4(tf.template at<LF>(Z), z);
       }
     } else {
-      z = wmm<C, F, false, false, LF, LS>(z, XQ + 16 * tf.it * LF, W1 + 16 * tf.jt);
+      z = wmm<WideFree<C>, F, false, false, LF, LS>(z, XQ + 16 * tf.it * LF, W1 + 16 * tf.jt);
       __syncthreads();
-      z = wmm<C, K, false, false, LK, LF>(z, C1 + 16 * tf.it * LK, G2 + 16 * tf.jt);
+      z = wmm<WideFree<C>, K, false, false, LK, LF>(z, C1 + 16 * tf.it * LK, G2 + 16 * tf.jt);
       stf4(tf.template at<LF>(Z), z);
     }
     __syncthreads();
