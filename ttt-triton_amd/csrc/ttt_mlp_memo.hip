@@ -282,8 +282,15 @@ __host__ __device__ __forceinline__ size_t memo_row_tile0(int NC, int M, int j) 
   return (size_t)j * NC - (size_t)M * j * (j + 1) / 2;
 }
 
-template <typename T, int FT, int HTT, bool BWD, bool PK, int NTW>
+// What memo_combine_kernel forms: the output, the output and the kept rows, or the
+// gate gradients.  Keeping is its own instantiation: as a run-time branch its
+// addresses spilled 11 registers of the plain forward (bf16 F64 FF256, B16 H12
+// T2048 M8: 537 -> 574 us; F32 FF64, a wave per SIMD fewer: 122 -> 151).
+enum class MemoPass { kOut, kOutRows, kGateGrads };
+
+template <typename T, int FT, int HTT, MemoPass PASS, bool PK, int NTW>
 __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoParams p) {
+  constexpr bool BWD = PASS == MemoPass::kGateGrads, KEEP = PASS == MemoPass::kOutRows;
   constexpr int F = 16 * FT;
   constexpr int FF = 16 * HTT;
   constexpr int K = 16;
@@ -313,8 +320,8 @@ __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoPa
   const T* __restrict__ XQ = static_cast<const T*>(p.XQ) + xoff;
   float* __restrict__ gb = p.gates + (size_t)chain * L.stride;
   const size_t ctiles = memo_row_tile0(NC, M, NS - 1);  // kept tiles of a chain
-  float* const rows = !BWD && p.rows != nullptr ? p.rows + chain * ctiles * (16 * F) : nullptr;
-  float* const rstds = !BWD && p.rows != nullptr ? p.rows + p.B * p.H * ctiles * (16 * F) + chain * ctiles * 16 : nullptr;
+  float* const rows = KEEP ? p.rows + chain * ctiles * (16 * F) : nullptr;
+  float* const rstds = KEEP ? p.rows + p.B * p.H * ctiles * (16 * F) + chain * ctiles * 16 : nullptr;
 
 #pragma unroll 1
   for (int half = 0; half < 2; ++half) {
@@ -456,7 +463,7 @@ __global__ __launch_bounds__(64 * kMemoWaves) void memo_combine_kernel(MlpMemoPa
           const float gr = gjv[t] * rstd;
 #pragma unroll
           for (int c = 0; c < FT; ++c) oacc[t][c] += gr * acc[t][c].v;
-          if (rows != nullptr) {  // lane order, past the caches: read once, by the backward
+          if constexpr (KEEP) {  // lane order, past the caches: read once, by the backward
             const size_t i = memo_row_tile0(NC, M, jm) + (t0 + t - (jm + 1) * M);
 #pragma unroll
             for (int c = 0; c < FT; ++c)
@@ -722,24 +729,24 @@ __global__ __launch_bounds__(kSegThreads) void memo_dxk_kernel(MlpMemoParams p) 
 }
 
 // ------------------------------------------------------------------ launchers
-template <typename T, int FT, int HTT, bool BWD, int NTW>
+template <typename T, int FT, int HTT, MemoPass PASS, int NTW>
 static hipError_t launch_combine_n(const MlpMemoParams& p, hipStream_t stream) {
   const dim3 grid(p.B * p.H * ((p.nchunk + 1) / 2)), block(64 * kMemoWaves);
   if constexpr (sizeof(T) == 2) {
     if (p.packed != nullptr) {
-      hipLaunchKernelGGL((memo_combine_kernel<T, FT, HTT, BWD, true, NTW>), grid, block, 0, stream, p);
+      hipLaunchKernelGGL((memo_combine_kernel<T, FT, HTT, PASS, true, NTW>), grid, block, 0, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((memo_combine_kernel<T, FT, HTT, BWD, false, NTW>), grid, block, 0, stream, p);
+  hipLaunchKernelGGL((memo_combine_kernel<T, FT, HTT, PASS, false, NTW>), grid, block, 0, stream, p);
   return hipGetLastError();
 }
 
-template <typename T, int FT, int HTT, bool BWD>
+template <typename T, int FT, int HTT, MemoPass PASS>
 static hipError_t launch_combine(const MlpMemoParams& p, hipStream_t stream) {
   // p.nchunk was set from the same chunk size
-  if (mlp_memo_chunk_tiles(p.B, p.H, p.NC) == kMemoWaves) return launch_combine_n<T, FT, HTT, BWD, 1>(p, stream);
-  return launch_combine_n<T, FT, HTT, BWD, kMemoTilesPerWave>(p, stream);
+  if (mlp_memo_chunk_tiles(p.B, p.H, p.NC) == kMemoWaves) return launch_combine_n<T, FT, HTT, PASS, 1>(p, stream);
+  return launch_combine_n<T, FT, HTT, PASS, kMemoTilesPerWave>(p, stream);
 }
 
 template <typename T, int FT, int HTT>
@@ -748,7 +755,7 @@ static hipError_t launch_memo_t(const MlpMemoParams& p, bool bwd, hipStream_t st
   if (bwd) {
     hipError_t e = hipSuccess;
     if (p.rows == nullptr) {
-      e = launch_combine<T, FT, HTT, true>(p, stream);
+      e = launch_combine<T, FT, HTT, MemoPass::kGateGrads>(p, stream);
     } else if (p.NC > p.M) {
       const long long tiles = (long long)p.B * p.H * (p.NC - p.M);
       hipLaunchKernelGGL((memo_dgam_kernel<T, FT>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, stream, p);
@@ -774,7 +781,8 @@ static hipError_t launch_memo_t(const MlpMemoParams& p, bool bwd, hipStream_t st
       if (e != hipSuccess) return e;
     }
   }
-  return launch_combine<T, FT, HTT, false>(p, stream);
+  if (p.rows != nullptr) return launch_combine<T, FT, HTT, MemoPass::kOutRows>(p, stream);
+  return launch_combine<T, FT, HTT, MemoPass::kOut>(p, stream);
 }
 
 template <typename T, int FT>
