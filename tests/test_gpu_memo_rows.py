@@ -62,6 +62,37 @@ def test_past_the_bound(monkeypatch):
         assert torch.equal(a, b)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,NC,F_,FF,M,kept", [
+    (4, 8, 61, 64, 64, 4, 10),   # 16 bits, rows past the caches: not kept below 128 hidden units
+    (4, 8, 61, 32, 128, 4, 7),   # kept from there on, with the images
+])
+def test_the_form_that_training_takes(B, H, NC, F_, FF, M, kept):
+    from ttt_amd import memo
+    d = {k: v.cuda() for k, v in _inputs(B, H, NC, F_, FF, M, seed=3, dtype=BF16).items()}
+    leaf = {k: d[k].detach().clone().requires_grad_(k in GRADS) for k in KEYS}
+    out = memo.mlp_memo_combine(*(leaf[k] for k in KEYS), M)
+    assert len(out.grad_fn.saved_tensors) == kept
+    grads = torch.autograd.grad(out, [leaf[k] for k in GRADS], d["dOut"])
+    out0, gates0 = memo.memo_combine_forward(*(d[k] for k in KEYS), M, images=False)
+    xq, xk, xu, xqw, *ws, lw, lb = (d[k] for k in KEYS)
+    ref = memo.memo_combine_backward(xq, xu, xqw, *ws, lw, lb, M, gates0, d["dOut"])
+    for a, b in zip((out, *grads), (out0, *ref)):
+        assert torch.equal(a, b)
+
+
+def test_training_form():
+    """16 bits keep the rows from 128 hidden units on or where the caches hold
+    them, fp32 always; the images are written unless cached rows are kept."""
+    from ttt_amd.memo import ROWS_CACHED_BYTES, training_form
+    cached, past = ROWS_CACHED_BYTES // 4, ROWS_CACHED_BYTES // 4 + 1
+    for dt in (F32, BF16, F16):
+        for FF in (32, 64, 128, 256):
+            assert training_form(0, FF, dt) == (False, True)
+            assert training_form(cached, FF, dt) == (True, False)
+            assert training_form(past, FF, dt) == (dt == F32 or FF >= 128, True)
+
+
 def test_rows_bytes_and_validation():
     from ttt_amd import _lib, memo
     lib = _lib.load()

@@ -112,13 +112,32 @@ def memo_combine_backward(XQ, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w,
 # The kept rows grow with the square of the sequence: past this, the backward
 # forms the readouts again.
 ROWS_MAX_BYTES = 1 << 30
+# Rows of this size stay in the caches on their way to the backward.
+ROWS_CACHED_BYTES = 16 << 20
 
 
 def memo_rows(B: int, H: int, NC: int, K: int, F: int, M: int) -> int:
-    """Floats of the readouts' rows that a training forward keeps, 0
+    """Floats of the readouts' rows that a training forward can keep, 0
     where there are none or they pass ROWS_MAX_BYTES."""
     n = _lib.load().ttt_mlp_memo_rows_bytes(B, H, NC, K, F, M)
     return n // 4 if n <= ROWS_MAX_BYTES else 0
+
+
+def training_form(rows: int, FF: int, dtype: torch.dtype):
+    """(whether a training forward keeps its `rows` floats of rows, whether it
+    writes the memo states' images).  A kept row is written and read once instead
+    of being formed again, which costs F FF products and FF GELUs: in fp32 the
+    rows are the cheaper at every size, in 16 bits from 128 hidden units on, and
+    below that only while the caches hold them.  Forward + backward, us, rows formed again (with
+    images) / kept without images / kept with images:
+      B16 H12 T2048 M8 bf16: F64 FF32 371/533/523, FF64 480/588/549, FF128 654/664/646,
+                             FF256 1,018/881/868; F32 FF32 209/264/249, FF64 268/290/276, FF128 400/372/356
+      B8 H12 T1024 M2 bf16:  F64 FF64 271/319/281, FF128 399/422/376
+      B1 H4 T1024 M8 bf16:   F64 FF64 66/55/56, FF256 104/75/76; F32 FF32 47/44/44
+      B16 H12 T2048 M8 fp32: F64 FF32 790/774, FF256 3,704/2,216; F32 FF32 482/424."""
+    small = 4 * rows <= ROWS_CACHED_BYTES
+    keep = rows > 0 and (dtype == torch.float32 or FF >= 128 or small)
+    return keep, not (keep and small)
 
 
 def memo_combine_backward_kept(XQ, XU, XQW, ln_w, ln_b, M: int, gates, rows, dout):
@@ -143,13 +162,15 @@ class MemoCombineFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M, eps=READOUT_EPS):
-        # the memo-state images pay off only when the backward stages the states too
-        training = any(ctx.needs_input_grad[1:4])
-        n = memo_rows(*XQ.shape, int(M)) if training and XQ.dim() == 5 and int(M) > 0 else 0
-        rows = torch.empty(n, device=XQ.device, dtype=torch.float32) if n else None
+        # an inference call writes neither rows nor images
+        keep = images = False
+        if any(ctx.needs_input_grad[1:4]):
+            n = memo_rows(*XQ.shape, int(M)) if XQ.dim() == 5 and int(M) > 0 else 0
+            keep, images = training_form(n, W1_memo.shape[-1], XQW.dtype)
+        rows = torch.empty(n, device=XQ.device, dtype=torch.float32) if keep else None
         out, gates = memo_combine_forward(XQ, XK, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, M, eps,
-                                          images=training and not n, rows=rows)
-        if n:
+                                          images=images, rows=rows)
+        if keep:
             ctx.save_for_backward(XQ, XU, XQW, ln_w, ln_b, gates, rows)
         else:
             ctx.save_for_backward(XQ, XU, XQW, W1_memo, b1_memo, W2_memo, b2_memo, ln_w, ln_b, gates)
