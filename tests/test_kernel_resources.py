@@ -49,3 +49,8 @@ def test_combiner_without_kept_rows(kernels, T, F_, FF, vgprs, spilled):
     name = f"memo_combine_kernelI{T}Li{F_ // 16}ELi{FF // 16}ELNS_8MemoPassE0ELb0ELi2E"
     (k,) = [r for n, r in kernels if name in n]
     assert k["vgpr_count"] <= vgprs and k["vgpr_spill_count"] <= spilled
+
+
+@pytest.mark.parametrize("kernel", ["wave16_fwd_state_kernel", "wave16_bwd_state_kernel"])
+def test_fp32_kernels_in_the_fp32_object_alone(kernels, kernel):
+    assert sum(kernel in n for n, _ in kernels) == 1

@@ -64,9 +64,10 @@ __device__ __forceinline__ unsigned w16_eta(const WideArgs& a, size_t m, int tok
   return wide_eta_last_raw<float, 16>(a, m, tok);
 }
 
-__global__ __launch_bounds__(kW16Threads) void wave16_fwd_state_kernel(WideArgs a) {
+// (templates: compiled where they are launched, in the fp32 translation unit)
+template <class C> __global__ __launch_bounds__(kW16Threads) void wave16_fwd_state_kernel(WideArgs a) {
   constexpr int K = 16, F = 64, FF = 256;
-  using Sl = WideSlot<W16>;
+  using Sl = WideSlot<C>;
   __shared__ __align__(16) float part[kW16Waves][16][kRowLd];  // a wave's W2 rows, then its share of Z2
   __shared__ __align__(16) float xk[2][16][kRowLd], xkT[2][F][kColLd];
   __shared__ __align__(16) float g2[16][kRowLd], u2T[F][kColLd];
@@ -267,9 +268,9 @@ __global__ __launch_bounds__(kW16Threads) void wave16_fwd_state_kernel(WideArgs 
 // wide_bwd_state_kernel), carrying dW1 [feature 16i + 4g + j][unit n] and dW2^T
 // [feature 16c + 4g + j][unit n].  Their products over units take operands that
 // pass through the wave's own rows in LDS.
-__global__ __launch_bounds__(kW16Threads) void wave16_bwd_state_kernel(WideArgs a) {
+template <class C> __global__ __launch_bounds__(kW16Threads) void wave16_bwd_state_kernel(WideArgs a) {
   constexpr int K = 16, F = 64, FF = 256;
-  using Sl = WideSlot<W16>;
+  using Sl = WideSlot<C>;
   __shared__ __align__(16) float part[kW16Waves][16][kRowLd];
   __shared__ __align__(16) float xk[16][kRowLd], g2[16][kRowLd], dz2[16][kRowLd];
   __shared__ __align__(16) float xkT[F][kColLd], g2T[F][kColLd], dz2T[F][kColLd];

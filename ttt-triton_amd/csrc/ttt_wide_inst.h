@@ -9,7 +9,7 @@ namespace {
 
 template <typename T, class C> hipError_t wide_fwd(const WideArgs& a, int chains, hipStream_t stream) {
   if constexpr (std::is_same_v<C, W16>)
-    hipLaunchKernelGGL(wave16_fwd_state_kernel, dim3(chains), dim3(kW16Threads), 0, stream, a);
+    hipLaunchKernelGGL(wave16_fwd_state_kernel<C>, dim3(chains), dim3(kW16Threads), 0, stream, a);
   else
     hipLaunchKernelGGL((wide_fwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
   hipLaunchKernelGGL((wide_fwd_readout_kernel<T, C>), dim3(chains * a.NC), dim3(C::NTH), 0, stream, a);
@@ -18,7 +18,7 @@ template <typename T, class C> hipError_t wide_fwd(const WideArgs& a, int chains
 template <typename T, class C> hipError_t wide_bwd(const WideArgs& a, int chains, hipStream_t stream) {
   hipLaunchKernelGGL((wide_bwd_readout_kernel<T, C>), dim3(chains * a.NC), dim3(C::NTH), 0, stream, a);
   if constexpr (std::is_same_v<C, W16>)
-    hipLaunchKernelGGL(wave16_bwd_state_kernel, dim3(chains), dim3(kW16Threads), 0, stream, a);
+    hipLaunchKernelGGL(wave16_bwd_state_kernel<C>, dim3(chains), dim3(kW16Threads), 0, stream, a);
   else
     hipLaunchKernelGGL((wide_bwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
   return hipGetLastError();
