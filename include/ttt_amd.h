@@ -59,13 +59,18 @@ enum ttt_eta_rule { TTT_ETA_DENSE = 0, TTT_ETA_LAYER = 1, TTT_ETA_CAUSAL = 2, TT
  * with TTT_DTYPE_F32 where ttt_split_saved_bytes is not 0: the split form,
  * whose per-chain launch carries the state alone and whose readout (and its
  * gradients) is a second launch with a workgroup per (chain, mini-batch).
- * Faster where few chains leave the GPU idle.  It takes a `saved` buffer of
- * ttt_split_saved_bytes in every call (the backward reads and writes the
- * forward's), no checkpoints, final state or workspace in the backward.
+ * Faster where few chains leave the GPU idle.  It takes a `saved` buffer in
+ * every call, of ttt_split_saved_bytes or as TTT_SAVED_SLOTS has it, and no
+ * checkpoints or final state in the backward.
+ *
+ * TTT_SAVED_SLOTS (where ttt_slots_bytes is not 0; both directions alike):
+ * `saved` is ttt_slots_bytes long, what a forward alone needs, about half of
+ * the whole, and the backward takes a workspace as long as the whole
+ * (ttt_linear_bwd_ws, ttt_mlp_bwd), into which it copies the slots first.
  *
  * TTT_STATE_SHARED (forwards only): W1_init, b1_init (W2_init, b2_init) are [H,...],
  * the same for every sequence of the batch, and read in place. */
-enum ttt_form { TTT_FORM_SPLIT = 0x100, TTT_STATE_SHARED = 0x200 };
+enum ttt_form { TTT_FORM_SPLIT = 0x100, TTT_STATE_SHARED = 0x200, TTT_SAVED_SLOTS = 0x400 };
 
 enum ttt_status {
   TTT_OK = 0,
@@ -112,9 +117,10 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
 /* Bytes of the saved buffer of ttt_linear_fwd / ttt_linear_bwd: with the
  * specialised kernels B*H*NC mini-batches x (3 * F * 64 + 256); with the
  * general-shape kernels, per chain, the state entering every mini-batch and
- * the fp32 scratch of one mini-batch; with K in {32, 48, 64} and F = 64, per
- * mini-batch, the state entering it (F F + F), 4 K F of forward values and of
- * the backward's handoff, F F + 3 F + 2 K more of the handoff, all fp32; 0 for
+ * the fp32 scratch of one mini-batch; with K in {32, 48, 64} and F = 64, while
+ * the slots stay within 4 GiB (past that the general-shape kernels run), per
+ * mini-batch a slot of the state entering it (F F + F) and 2 K F + K of forward
+ * values, and 2 K F + F F + 3 F + K of the backward's handoff, all fp32; 0 for
  * unsupported sizes. */
 size_t ttt_linear_saved_bytes(int B, int H, int NC, int K, int F);
 
@@ -122,6 +128,12 @@ size_t ttt_linear_saved_bytes(int B, int H, int NC, int K, int F);
  * Linear loop): K = 16 with F = 64 (MLP: FF = 64 or 256, or F = 32 with FF =
  * 128); 0 for any other shape. */
 size_t ttt_split_saved_bytes(int B, int H, int NC, int K, int F, int FF);
+
+/* Bytes of `saved` with TTT_SAVED_SLOTS, for the kernels with a slot per
+ * mini-batch (K in {32, 48, 64} above, and with `split` the split form; FF = 0:
+ * the Linear loop): the slots without the backward's handoff, and a final state
+ * per chain.  0 for any other problem. */
+size_t ttt_slots_bytes(int B, int H, int NC, int K, int F, int FF, int split);
 
 /* TTT-Linear backward: gradients of sum(out * dout) wrt every input, the
  * final state's gradient taken as zero (the ops path discards W_last).
@@ -143,6 +155,16 @@ int ttt_linear_bwd(const void* XQ, const void* XK, const void* XV, const void* e
                    const void* dout, int B, int H, int NC, int K, int F, int G, int dtype, int eta_rule, float eps,
                    void* dXQ, void* dXK, void* dXV, void* deta, float* dW1, float* db1,
                    float* dln_w, float* dln_b, const void* saved, size_t saved_bytes, void* stream);
+
+/* The same with a workspace, workspace_bytes >= ttt_linear_saved_bytes(...)
+ * (ttt_split_saved_bytes in the split form), where TTT_SAVED_SLOTS is set; unused
+ * otherwise (it may be NULL then). */
+int ttt_linear_bwd_ws(const void* XQ, const void* XK, const void* XV, const void* eta,
+                      const float* ln_w, const float* ln_b, const float* W1_ckpt, const float* W1_last,
+                      const void* dout, int B, int H, int NC, int K, int F, int G, int dtype, int eta_rule, float eps,
+                      void* dXQ, void* dXK, void* dXV, void* deta, float* dW1, float* db1,
+                      float* dln_w, float* dln_b, const void* saved, size_t saved_bytes,
+                      void* workspace, size_t workspace_bytes, void* stream);
 
 /* TTT-MLP forward (2-layer GELU(tanh) fast-weight MLP) over all NC
  * mini-batches.  Replaces ttt_mlp_scan_forward (kernels/mlp_forward.py:6-237)
@@ -178,8 +200,10 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
  * + (FF + F) * 4 + 3 * F * 64 + 4096); with the general-shape kernels, per
  * chain, the state entering every mini-batch and the fp32 scratch of one
  * mini-batch; with K in {32, 48, 64} and (F, FF) one of (64, 64), (64, 256)
- * and (32, 128), per mini-batch, twice the state (2 F FF + FF + F), 4 K (FF + F)
- * of forward values and of the backward's handoff, and 2 F + 2 K, all fp32. */
+ * and (32, 128), while the slots stay within 4 GiB (past that the general-shape
+ * kernels run), per mini-batch a slot of the state entering it (2 F FF + FF + F)
+ * and 2 K (FF + F) + K of forward values, and as much and 2 F more of the
+ * backward's handoff, all fp32. */
 size_t ttt_mlp_saved_bytes(int B, int H, int NC, int K, int F, int FF, int dtype);
 
 /* Bytes of device workspace ttt_mlp_bwd uses: B*H*NC mini-batches x
@@ -189,7 +213,7 @@ size_t ttt_mlp_saved_bytes(int B, int H, int NC, int K, int F, int FF, int dtype
  * 48 KB at K = 64 (less at smaller K), the handoff of their two-launch form,
  * which they use when given that much and otherwise run in one launch with
  * at least 256 bytes; 256 with the other general shapes, which keep their
- * scratch in `saved`. */
+ * scratch in `saved` (with TTT_SAVED_SLOTS ttt_mlp_saved_bytes, or ttt_split_saved_bytes). */
 size_t ttt_mlp_bwd_workspace_bytes(int B, int H, int NC, int K, int F, int FF, int dtype);
 
 /* TTT-MLP backward: gradients of sum(out * dout) wrt every input (final

@@ -29,6 +29,12 @@ bool take_split(int& eta_rule) {
   eta_rule &= ~TTT_FORM_SPLIT;
   return split;
 }
+// the same of TTT_SAVED_SLOTS
+bool take_slots(int& eta_rule) {
+  const bool slots = (eta_rule & TTT_SAVED_SLOTS) != 0;
+  eta_rule &= ~TTT_SAVED_SLOTS;
+  return slots;
+}
 // the same of TTT_STATE_SHARED: the number of distinct initial states
 int take_states(int& eta_rule, int B, int H) {
   const bool shared = (eta_rule & TTT_STATE_SHARED) != 0;
@@ -92,6 +98,11 @@ int hip_status(hipError_t e) { return e == hipSuccess ? TTT_OK : TTT_ERR_HIP; }
 // Shapes of the specialised inner-loop kernels (16-token mini-batches held in
 // registers); every other valid shape takes the general-shape kernels.
 bool fast_linear_shape(int K, int F) { return K == 16 && (F == 32 || F == 64); }
+// (FF = 0: the Linear loop)
+bool wide_takes(int B, int H, int NC, int K, int F, int FF, bool split) {
+  return split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) != 0
+               : ttt::wide_runs(B, H, NC, K, F, FF > 0 ? FF : F, FF > 0);
+}
 bool fast_mlp_shape(int K, int F, int FF) {
   return fast_linear_shape(K, F) && (FF == 64 || FF == 128 || FF == 256);
 }
@@ -152,16 +163,17 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
                    float* W1_ckpt, float* b1_ckpt, void* saved, size_t saved_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
-  const bool split = take_split(eta_rule);
+  const bool split = take_split(eta_rule), slots = take_slots(eta_rule);
   const int NI = take_states(eta_rule, B, H);
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
   eta_rule = eta_rule_of(eta_rule, dtype);
   const bool fast = fast_linear_shape(K, F) && !split;
   st = fast ? check_linear(NC, F) : TTT_OK;
   if (st != TTT_OK) return st;
-  const size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, 0) : ttt_linear_saved_bytes(B, H, NC, K, F);
+  size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, 0) : ttt_linear_saved_bytes(B, H, NC, K, F);
   if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
   if (split && need == 0) return TTT_ERR_SHAPE;
+  if (slots && (need = ttt_slots_bytes(B, H, NC, K, F, 0, split)) == 0) return TTT_ERR_ARG;
   REQUIRE_PTR(XQ);
   REQUIRE_PTR(XK);
   REQUIRE_PTR(XV);
@@ -193,6 +205,7 @@ int ttt_linear_fwd(const void* XQ, const void* XK, const void* XV, const void* e
     q.W1_init = W1_init;
     q.b1_init = b1_init;
     q.NI = NI;
+    q.slots = slots;
     q.out = out;
     q.W1_last = W1_last;
     q.b1_last = b1_last;
@@ -246,17 +259,28 @@ int ttt_linear_bwd(const void* XQ, const void* XK, const void* XV, const void* e
                    int NC, int K, int F, int G, int dtype, int eta_rule, float eps, void* dXQ, void* dXK,
                    void* dXV, void* deta, float* dW1, float* db1, float* dln_w, float* dln_b, const void* saved,
                    size_t saved_bytes, void* stream) {
+  return ttt_linear_bwd_ws(XQ, XK, XV, eta, ln_w, ln_b, W1_ckpt, W1_last, dout, B, H, NC, K, F, G, dtype, eta_rule,
+                           eps, dXQ, dXK, dXV, deta, dW1, db1, dln_w, dln_b, saved, saved_bytes, nullptr, 0, stream);
+}
+
+int ttt_linear_bwd_ws(const void* XQ, const void* XK, const void* XV, const void* eta, const float* ln_w,
+                      const float* ln_b, const float* W1_ckpt, const float* W1_last, const void* dout, int B, int H,
+                      int NC, int K, int F, int G, int dtype, int eta_rule, float eps, void* dXQ, void* dXK,
+                      void* dXV, void* deta, float* dW1, float* db1, float* dln_w, float* dln_b, const void* saved,
+                      size_t saved_bytes, void* workspace, size_t workspace_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
-  const bool split = take_split(eta_rule);
+  const bool split = take_split(eta_rule), slots = take_slots(eta_rule);
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
   eta_rule = eta_rule_of(eta_rule, dtype);
   const bool fast = fast_linear_shape(K, F) && !split;
   st = fast ? check_linear(NC, F) : TTT_OK;
   if (st != TTT_OK) return st;
-  const size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, 0) : ttt_linear_saved_bytes(B, H, NC, K, F);
+  size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, 0) : ttt_linear_saved_bytes(B, H, NC, K, F);
   if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
   if (split && need == 0) return TTT_ERR_SHAPE;
+  const size_t full = need;
+  if (slots && (need = ttt_slots_bytes(B, H, NC, K, F, 0, split)) == 0) return TTT_ERR_ARG;
   REQUIRE_PTR(XQ);
   REQUIRE_PTR(XK);
   REQUIRE_PTR(XV);
@@ -279,8 +303,13 @@ int ttt_linear_bwd(const void* XQ, const void* XK, const void* XV, const void* e
   if (saved == nullptr) return TTT_ERR_WORKSPACE;
   if (!aligned16(saved)) return TTT_ERR_ALIGN;
   if (saved_bytes < need) return TTT_ERR_WORKSPACE;
+  if (slots) {
+    if (workspace == nullptr || workspace_bytes < full) return TTT_ERR_WORKSPACE;
+    if (!aligned16(workspace)) return TTT_ERR_ALIGN;
+  }
   if (!fast) {
     ttt::GenBwdParams q{};
+    q.spread = slots ? workspace : nullptr;
     q.XQ = XQ;
     q.XK = XK;
     q.XV = XV;
@@ -347,14 +376,14 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
                 float* b2_memo, void* saved, size_t saved_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
-  const bool split = take_split(eta_rule);
+  const bool split = take_split(eta_rule), slots = take_slots(eta_rule);
   const int NI = take_states(eta_rule, B, H);
   const bool fast = fast_mlp_shape(K, F, FF) && !split;
   if (!fast && !ttt::gen_shape_ok(K, F, FF, true)) return TTT_ERR_SHAPE;
-  const size_t need =
-      split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) : ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype);
+  size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) : ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype);
   if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
   if (split && need == 0) return TTT_ERR_SHAPE;
+  if (slots && (need = ttt_slots_bytes(B, H, NC, K, F, FF, split)) == 0) return TTT_ERR_ARG;
   st = fast ? check_mlp(NC, F, FF, dtype) : TTT_OK;
   if (st != TTT_OK) return st;
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
@@ -399,6 +428,7 @@ int ttt_mlp_fwd(const void* XQ, const void* XK, const void* XV, const void* eta,
     q.W2_init = W2_init;
     q.b2_init = b2_init;
     q.NI = NI;
+    q.slots = slots;
     q.out = out;
     q.W1_last = W1_last;
     q.b1_last = b1_last;
@@ -473,6 +503,11 @@ size_t ttt_split_saved_bytes(int B, int H, int NC, int K, int F, int FF) {
   return ttt::wide_saved_bytes(B, H, NC, K, F, FF > 0 ? FF : F, FF > 0);
 }
 
+size_t ttt_slots_bytes(int B, int H, int NC, int K, int F, int FF, int split) {
+  if (B <= 0 || H <= 0 || NC <= 0 || !wide_takes(B, H, NC, K, F, FF, split != 0)) return 0;
+  return ttt::wide_slots_bytes(B, H, NC, K, F, FF > 0 ? FF : F, FF > 0);
+}
+
 size_t ttt_mlp_saved_bytes(int B, int H, int NC, int K, int F, int FF, int dtype) {
   if (B <= 0 || H <= 0 || NC <= 0 || K <= 0 || F <= 0 || FF <= 0) return 0;
   if (!dtype_ok(dtype)) return 0;
@@ -513,13 +548,14 @@ static int mlp_bwd_impl(const void* XQ, const void* XK, const void* XV, const vo
                 size_t workspace_bytes, void* stream) {
   int st = check_common(B, H, NC, K, F, G, dtype, eps);
   if (st != TTT_OK) return st;
-  const bool split = take_split(eta_rule);
+  const bool split = take_split(eta_rule), slots = take_slots(eta_rule);
   const bool fast = fast_mlp_shape(K, F, FF) && !split;
   if (!fast && !ttt::gen_shape_ok(K, F, FF, true)) return TTT_ERR_SHAPE;
-  const size_t need =
-      split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) : ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype);
+  size_t need = split ? ttt_split_saved_bytes(B, H, NC, K, F, FF) : ttt_mlp_saved_bytes(B, H, NC, K, F, FF, dtype);
   if (split && dtype != TTT_DTYPE_F32) return TTT_ERR_DTYPE;
   if (split && need == 0) return TTT_ERR_SHAPE;
+  const size_t full = need;
+  if (slots && (need = ttt_slots_bytes(B, H, NC, K, F, FF, split)) == 0) return TTT_ERR_ARG;
   st = fast ? check_mlp(NC, F, FF, dtype) : TTT_OK;
   if (st != TTT_OK) return st;
   if (!eta_rule_ok(eta_rule)) return TTT_ERR_ARG;
@@ -536,13 +572,15 @@ static int mlp_bwd_impl(const void* XQ, const void* XK, const void* XV, const vo
   if (saved == nullptr) return TTT_ERR_WORKSPACE;
   if (!aligned16(saved)) return TTT_ERR_ALIGN;
   if (saved_bytes < need) return TTT_ERR_WORKSPACE;
-  if (!split) {
+  if (slots && workspace_bytes < full) return TTT_ERR_WORKSPACE;
+  if (!split || slots) {
     if (workspace == nullptr) return TTT_ERR_WORKSPACE;
     if (!aligned16(workspace)) return TTT_ERR_ALIGN;
     if (workspace_bytes < mlp_bwd_min_workspace(B, H, NC, K, F, FF, dtype)) return TTT_ERR_WORKSPACE;
   }
   if (!fast) {
     ttt::GenBwdParams q{};
+    q.spread = slots ? workspace : nullptr;
     q.ws = workspace;
     q.ws_bytes = workspace_bytes;
     q.XQ = XQ;

@@ -830,13 +830,13 @@ bool gen_shape_ok(int K, int F, int FF, bool mlp) {
 }
 
 size_t gen_saved_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp) {
-  if (wide_shape_ok(K, F, FF, mlp)) return wide_saved_bytes(B, H, NC, K, F, FF, mlp);
+  if (wide_runs(B, H, NC, K, F, FF, mlp)) return wide_saved_bytes(B, H, NC, K, F, FF, mlp);
   return (size_t)B * H * GenLayout(K, F, FF, NC, mlp).per_chain * sizeof(float);
 }
 
 hipError_t launch_gen_fwd(const GenFwdParams& q, int dtype, hipStream_t stream) {
   if (small_shape_ok(q.K, q.F, q.FF, q.mlp) && !gen_force_general()) return launch_small_fwd(q, dtype, stream);
-  if (wide_shape_ok(q.K, q.F, q.FF, q.mlp)) return launch_wide_fwd(q, dtype, stream);
+  if (wide_runs(q.B, q.H, q.NC, q.K, q.F, q.FF, q.mlp)) return launch_wide_fwd(q, dtype, stream);
   GenArgs a{};
   a.XQ = q.XQ;
   a.XK = q.XK;
@@ -872,7 +872,7 @@ hipError_t launch_gen_fwd(const GenFwdParams& q, int dtype, hipStream_t stream) 
 
 hipError_t launch_gen_bwd(const GenBwdParams& q, int dtype, hipStream_t stream) {
   if (small_shape_ok(q.K, q.F, q.FF, q.mlp) && !gen_force_general()) return launch_small_bwd(q, dtype, stream);
-  if (wide_shape_ok(q.K, q.F, q.FF, q.mlp)) return launch_wide_bwd(q, dtype, stream);
+  if (wide_runs(q.B, q.H, q.NC, q.K, q.F, q.FF, q.mlp)) return launch_wide_bwd(q, dtype, stream);
   GenArgs a{};
   a.XQ = q.XQ;
   a.XK = q.XK;

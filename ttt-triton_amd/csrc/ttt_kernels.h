@@ -233,6 +233,7 @@ struct GenFwdParams {
   float *W1_ckpt, *b1_ckpt, *W2_ckpt, *b2_ckpt;
   float *W1_memo, *b1_memo, *W2_memo, *b2_memo;
   void* saved;
+  bool slots;  // ttt_wide.h's kernels: `saved` holds the slots alone
   int B, H, NC, K, F, FF, G, M, eta_rule;
   bool mlp;
   float eps;
@@ -245,6 +246,7 @@ struct GenBwdParams {
   void* saved;  // written by the forward with the same shapes
   void* ws;     // the backward's workspace (the register-resident MLP backward's handoff), may be null
   size_t ws_bytes;
+  void* spread;  // ttt_wide.h's kernels where `saved` holds the slots alone: wide_saved_bytes, else null
   int B, H, NC, K, F, FF, eta_rule;
   bool mlp;
   float eps;
@@ -261,9 +263,12 @@ bool small_shape_ok(int K, int F, int FF, bool mlp);
 // (0 for K outside 16..64); a smaller workspace runs the one-launch form
 size_t small_mlp_bwd_hand_bytes(int B, int H, int NC, int K);
 // mini-batch-in-LDS kernels (ttt_wide.h) for K = 32, 48, 64 with F = 64 (MLP:
-// FF = 64 or 256, or F = 32 with FF = 128), their own slots in `saved`
-bool wide_shape_ok(int K, int F, int FF, bool mlp);
+// FF = 64 or 256, or F = 32 with FF = 128), up to a size.  `saved` is their own:
+// per mini-batch a slot with the place of the backward's handoff
+// (wide_saved_bytes), or without it (wide_slots_bytes)
+bool wide_runs(int B, int H, int NC, int K, int F, int FF, bool mlp);
 size_t wide_saved_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp);
+size_t wide_slots_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp);
 hipError_t launch_wide_fwd(const GenFwdParams& p, int dtype, hipStream_t stream);
 hipError_t launch_wide_bwd(const GenBwdParams& p, int dtype, hipStream_t stream);
 bool gen_force_general();  // TTT_OPT_SMALL_KERNELS = 0: always the staged general-shape kernels

@@ -65,7 +65,8 @@ __device__ __forceinline__ unsigned w16_eta(const WideArgs& a, size_t m, int tok
 }
 
 // (templates: compiled where they are launched, in the fp32 translation unit)
-template <class C> __global__ __launch_bounds__(kW16Threads) void wave16_fwd_state_kernel(WideArgs a) {
+// STRIDE: floats from one slot to the next (from the arguments: 325 -> 333 us at B3 H5, 37 mini-batches)
+template <class C, int STRIDE> __global__ __launch_bounds__(kW16Threads) void wave16_fwd_state_kernel(WideArgs a) {
   constexpr int K = 16, F = 64, FF = 256;
   using Sl = WideSlot<C>;
   __shared__ __align__(16) float part[kW16Waves][16][kRowLd];  // a wave's W2 rows, then its share of Z2
@@ -77,7 +78,7 @@ template <class C> __global__ __launch_bounds__(kW16Threads) void wave16_fwd_sta
   const int tid = threadIdx.x, l = tid & 63, g = l >> 4, n = l & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int NK = (NC + a.G - 1) / a.G, NS = (NC + a.M - 1) / a.M;
-  float* const slot0 = a.saved + chain * NC * (size_t)Sl::FLOATS;
+  float* const slot0 = a.saved + chain * NC * (size_t)STRIDE;
   const float lw = a.ln_w[(size_t)h * F + l], lb = a.ln_b[(size_t)h * F + l];
   float* const own = &part[w][0][0];
 
@@ -115,7 +116,7 @@ template <class C> __global__ __launch_bounds__(kW16Threads) void wave16_fwd_sta
   int ck = 0, ck_in = 0, mk = 0, mk_in = 1;
   auto emit = [&](int s) {  // the state entering mini-batch s
     if (s < NC) {
-      float* q = slot0 + (size_t)s * Sl::FLOATS;
+      float* q = slot0 + (size_t)s * STRIDE;
       put(q + Sl::W1, q + Sl::B1, q + Sl::W2, q + Sl::B2);
       if (ck_in == 0 && a.W1_ckpt != nullptr) {
         // (only W1's checkpoints are always there)
@@ -170,7 +171,7 @@ template <class C> __global__ __launch_bounds__(kW16Threads) void wave16_fwd_sta
     const int l = pinned(lane_id()), g = l >> 4, n = l & 15, tid = 64 * w + l;
     const int b = s & 1;
     const size_t m = pinned_index(chain * NC + s);
-    float* const slot = a.saved + m * Sl::FLOATS;
+    float* const slot = a.saved + m * STRIDE;
     float e_r = wide_eta_last_val<float, K>(a, er);
     f4 e4;
 #pragma unroll

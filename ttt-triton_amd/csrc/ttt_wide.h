@@ -31,7 +31,8 @@
 //
 // Everything is held and summed in fp32 whatever the activation type, as in
 // the general-shape kernels (ttt_generic.hip); activations are converted on
-// load.  `saved` holds one slot per (chain, mini-batch), WideSlot below.
+// load.  `saved` holds one slot per (chain, mini-batch), WideSlot below, with or
+// without the handoff's place in it.
 #pragma once
 
 #include "ttt_eta.h"
@@ -69,7 +70,12 @@ template <class C> struct WideFree {
   static constexpr bool PIN = false;
 };
 
-// floats of one (chain, mini-batch) slot of `saved`
+// floats of one (chain, mini-batch) slot of `saved`: what the forward writes, then
+// the handoff, which the backward writes.  A forward's `saved` may hold the first
+// part alone (half of it); a backward then begins with wide_spread_kernel.
+// (With the two parts at strides of their own the state launches of the backward
+// lost 3%: K = F = FF = 64, B32 H4, 8 mini-batches 166 -> 170 us, the split form's
+// F = 32, FF = 128, 64 chains, 32 mini-batches 313 -> 326.)
 template <class C> struct WideSlot {
   static constexpr int STATE = C::MLP ? 2 * C::F * C::FF + C::FF + C::F : C::F * C::F + C::F;
   // the state entering the mini-batch
@@ -84,10 +90,11 @@ template <class C> struct WideSlot {
   static constexpr int G2 = P + (C::MLP ? C::K * C::FF : 0);
   static constexpr int ZH = G2 + C::K * C::F;
   static constexpr int SIG = ZH + C::K * C::F;
+  static constexpr int FWD = SIG + C::K;
   // the handoff from wide_bwd_readout to wide_bwd_state: the readout's terms
   // of dG1, dX2, dG2, dXK, the state gradient, the LayerNorm parameters'
   // gradients, and deta's last row (for an lr rule: dlr)
-  static constexpr int HG1 = SIG + C::K;
+  static constexpr int HG1 = FWD;
   static constexpr int HX2 = HG1 + (C::MLP ? C::K * C::FF : 0);
   static constexpr int HG2 = HX2 + (C::MLP ? C::K * C::FF : 0);
   static constexpr int HXK = HG2 + C::K * C::F;
@@ -109,6 +116,9 @@ struct WideArgs {
   void *dXQ, *dXK, *dXV, *deta;
   float *dW1, *db1, *dW2, *db2, *dln_w, *dln_b;
   float* saved;
+  size_t slot_stride;   // (forward) floats from one slot to the next (backward: FLOATS)
+  float* fin;           // (forward) where the state after a chain's last mini-batch goes
+  size_t fin_stride;    // floats from one chain's to the next
   int H, NC, G, M, NI, eta_rule;
   float eps;
 };

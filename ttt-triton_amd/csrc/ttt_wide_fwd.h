@@ -57,7 +57,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
   const WideTile<C::FT> tf(w);    // its K x F tile
   const bool has_f = C::ALLF || w < C::KT * C::FT;
   const int NK = (NC + a.G - 1) / a.G, NS = (NC + a.M - 1) / a.M;
-  float* const slot0 = a.saved + chain * NC * (size_t)Sl::FLOATS;
+  float* const slot0 = a.saved + chain * NC * a.slot_stride;
 
   const size_t ic = chain % (size_t)a.NI;
   f4 w1[NSL][NT], w2[NSL][NT];
@@ -88,9 +88,9 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
     auto at = [](float* p, size_t k, size_t n) { return p != nullptr ? p + k * n : nullptr; };
     WideStateDst d{nullptr, nullptr, nullptr, nullptr};
     if (i == 0) {
-      // (a store on every path, so that the waits for loads can count past it;
-      // after the last mini-batch it goes where the backward will write)
-      float* q = s < NC ? slot0 + (size_t)s * Sl::FLOATS : slot0 + (size_t)(NC - 1) * Sl::FLOATS + Sl::HST;
+      // (a store on every path, so that the waits for loads can count past it:
+      // after the last mini-batch too)
+      float* q = s < NC ? slot0 + s * a.slot_stride : a.fin + chain * a.fin_stride;
       d = WideStateDst{q + Sl::W1, q + Sl::B1, q + Sl::W2, q + Sl::B2};
     } else if (i == 1 && s < NC && ck_in == 0) {
       const size_t k = chain * NK + ck;
@@ -181,7 +181,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
 
   for (int s = 0; s < NC; ++s) {
     float* const XKs = sm + (s & 1) * C::SLOT;
-    float* const slot = slot0 + (size_t)s * Sl::FLOATS;
+    float* const slot = slot0 + s * a.slot_stride;
     next_dst();
     f4 x2[MLP ? NSL : 1], d1[MLP ? NSL : 1];
     f4 z2 = f4{0.f, 0.f, 0.f, 0.f};
@@ -486,7 +486,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
   __shared__ __align__(16) float sm[WideReadout<T, C>::LDS];
   const size_t m = blockIdx.x;  // chain * NC + s
   const int h = (int)((m / (size_t)a.NC) % (size_t)a.H);
-  WideReadout<T, C> ro(sm, a.saved + m * WideSlot<C>::FLOATS);
+  WideReadout<T, C> ro(sm, a.saved + m * a.slot_stride);
   ro.forward(a, m);
   float sd;
   const typename VecF<V>::type xh = ro.norm(a.eps, sd);

@@ -8,9 +8,13 @@ namespace ttt {
 namespace {
 
 template <typename T, class C> hipError_t wide_fwd(const WideArgs& a, int chains, hipStream_t stream) {
-  if constexpr (std::is_same_v<C, W16>)
-    hipLaunchKernelGGL(wave16_fwd_state_kernel<C>, dim3(chains), dim3(kW16Threads), 0, stream, a);
-  else
+  using Sl = WideSlot<C>;
+  if constexpr (std::is_same_v<C, W16>) {
+    if (a.slot_stride == Sl::FLOATS)
+      hipLaunchKernelGGL((wave16_fwd_state_kernel<C, Sl::FLOATS>), dim3(chains), dim3(kW16Threads), 0, stream, a);
+    else
+      hipLaunchKernelGGL((wave16_fwd_state_kernel<C, Sl::FWD>), dim3(chains), dim3(kW16Threads), 0, stream, a);
+  } else
     hipLaunchKernelGGL((wide_fwd_state_kernel<T, C>), dim3(chains), dim3(C::NTH), 0, stream, a);
   hipLaunchKernelGGL((wide_fwd_readout_kernel<T, C>), dim3(chains * a.NC), dim3(C::NTH), 0, stream, a);
   return hipGetLastError();

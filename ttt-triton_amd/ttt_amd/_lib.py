@@ -6,6 +6,7 @@ library is missing or fails to load, every entry point raises."""
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -29,6 +30,7 @@ ETA_CAUSAL = 2
 ETA_DENSE_F32 = 3  # dense eta kept in fp32 under 16-bit activations (chosen from eta's dtype)
 FORM_SPLIT = 0x100  # or'ed into the eta rule: the state and the readout as two launches
 STATE_SHARED = 0x200  # (forward): initial states [H,...], one for every sequence
+SAVED_SLOTS = 0x400  # `saved` without the place of the backward's handoff (slot_saved below)
 ETA_RULES = {"dense": ETA_DENSE, "layer": ETA_LAYER, "causal": ETA_CAUSAL}
 
 # process-wide options (enum ttt_option)
@@ -52,9 +54,11 @@ SIGNATURES = {
     "ttt_linear_fwd": (_I, [_P] * 8 + [_I] * 8 + [_F] + [_P] * 5 + [_P, _S, _P]),
     "ttt_linear_saved_bytes": (_S, [_I] * 5),
     "ttt_linear_bwd": (_I, [_P] * 9 + [_I] * 8 + [_F] + [_P] * 8 + [_P, _S, _P]),
+    "ttt_linear_bwd_ws": (_I, [_P] * 9 + [_I] * 8 + [_F] + [_P] * 8 + [_P, _S, _P, _S, _P]),
     "ttt_mlp_fwd": (_I, [_P] * 10 + [_I] * 10 + [_F] + [_P] * 13 + [_P, _S, _P]),
     "ttt_mlp_saved_bytes": (_S, [_I] * 7),
     "ttt_split_saved_bytes": (_S, [_I] * 6),
+    "ttt_slots_bytes": (_S, [_I] * 7),
     "ttt_mlp_bwd_workspace_bytes": (_S, [_I] * 7),
     "ttt_mlp_bwd": (_I, [_P] * 15 + [_I] * 9 + [_F] + [_P] * 10 + [_P, _S, _P, _S, _P]),
     "ttt_mlp_bwd_noalloc": (_I, [_P] * 15 + [_I] * 9 + [_F] + [_P] * 10 + [_P, _S, _P]),
@@ -123,7 +127,38 @@ def fast_mlp_shape(K: int, F: int, FF: int) -> bool:
     return fast_linear_shape(K, F) and FF in (64, 128, 256)
 
 
-# The split form's `saved` buffer is bounded: it holds every mini-batch's state.
+# A training forward's `saved` has the place of the backward's handoff up to this
+# size; past it, and in inference, it holds the slots alone, and the backward
+# copies them into a buffer of its own first.
+SLOTS_WITH_HANDOFF_BYTES = 1 << 30
+
+
+@functools.lru_cache(maxsize=1024)
+def slot_bytes(B: int, H: int, NC: int, K: int, F: int, FF: int, split: bool):
+    """Where a mini-batch has a slot (FF = 0: the Linear loop): the bytes of `saved`
+    with the place of the handoff, and of the slots alone; 0 elsewhere."""
+    lib = load()
+    slots = lib.ttt_slots_bytes(B, H, NC, K, F, FF, split)
+    if not slots:
+        return 0, 0
+    full = (lib.ttt_split_saved_bytes(B, H, NC, K, F, FF) if split else
+            lib.ttt_mlp_saved_bytes(B, H, NC, K, F, FF, 0) if FF else lib.ttt_linear_saved_bytes(B, H, NC, K, F))
+    return full, slots
+
+
+def slot_saved(*shape_split, train: bool):
+    """(bytes of `saved`, SAVED_SLOTS or 0) of a forward, (0, 0) where no mini-batch has a slot."""
+    full, slots = slot_bytes(*shape_split)
+    return (slots, SAVED_SLOTS if slots else 0) if not train or full > SLOTS_WITH_HANDOFF_BYTES else (full, 0)
+
+
+def slot_workspace(saved, *shape_split):
+    """(bytes of the backward's workspace, SAVED_SLOTS or 0) given the forward's `saved`."""
+    full, slots = slot_bytes(*shape_split)
+    return (full, SAVED_SLOTS) if slots and saved.numel() == slots else (0, 0)
+
+
+# The split form's `saved` buffer and handoff are bounded: they hold every mini-batch's state.
 SPLIT_MAX_BYTES = 1 << 30
 
 

@@ -47,12 +47,11 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
     by eta_rule "layer" or "causal".  Returns (out [B,H,NC,K,F] in XQ.dtype,
     (W1_ckpt, b1_ckpt) or None, (W1_last, b1_last) or None, saved or None).
 
-    `saved` (uint8, ttt_linear_saved_bytes long) holds what linear_backward
-    reads instead of re-running the forward; the backward needs it together
-    with W1_ckpt and W1_last.  With `split` (fp32, K = 16, F = 64) the state and the
-    readout run as two launches (TTT_FORM_SPLIT): the buffer is then
-    ttt_split_saved_bytes long, always allocated, and all that a split backward
-    needs."""
+    `saved` (uint8, ttt_linear_saved_bytes long, or ttt_slots_bytes as
+    _lib.slot_saved has it) holds what linear_backward reads instead of re-running
+    the forward; the backward needs it together with W1_ckpt and W1_last.  With `split` (fp32, K = 16,
+    F = 64) the state and the readout run as two launches (TTT_FORM_SPLIT): the
+    buffer is then always allocated, and all that a split backward needs."""
     rule = _lib.eta_rule_code(eta_rule)
     B, H, NC, K, F = _check_shapes(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, rule)
     dev = check_device(XQ, XK, XV, eta, W1, b1, ln_w, ln_b)
@@ -78,10 +77,11 @@ def linear_forward(ln_w, ln_b, W1, b1, XQ, XV, XK, eta, G: int, eps: float = LN_
     saved = None
     if split:
         krule |= _lib.FORM_SPLIT
-    if want_saved or split or not _lib.fast_linear_shape(K, F):
-        nbytes = (lib.ttt_split_saved_bytes(B, H, NC, K, F, 0) if split
-                  else lib.ttt_linear_saved_bytes(B, H, NC, K, F))
-        saved = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    general = split or not _lib.fast_linear_shape(K, F)
+    if want_saved or general:
+        nbytes, form = _lib.slot_saved(B, H, NC, K, F, 0, split, train=want_saved) if general else (0, 0)
+        krule |= form
+        saved = torch.empty(nbytes or lib.ttt_linear_saved_bytes(B, H, NC, K, F), device=dev, dtype=torch.uint8)
     with on_device(dev):
         st = lib.ttt_linear_fwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb), ptr(w1), ptr(bb),
@@ -123,13 +123,17 @@ def linear_backward(ln_w, ln_b, XQ, XV, XK, eta, W1_ckpt, W1_last, saved, dout, 
     dln = torch.empty((2, B, H, F), device=dev, dtype=torch.float32)
     dlw, dlb = dln
     lib = _lib.load()
+    general = split or not _lib.fast_linear_shape(K, F)
+    nws, form = _lib.slot_workspace(saved, B, H, NC, K, F, 0, split) if general else (0, 0)
+    krule |= form
+    ws = torch.empty(nws, device=dev, dtype=torch.uint8) if nws else None
     with on_device(dev):
-        st = lib.ttt_linear_bwd(
+        st = lib.ttt_linear_bwd_ws(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb),
             *(ptr(t) if t is not None else None for t in (W1_ckpt, W1_last)), ptr(do),
             B, H, NC, K, F, int(G), code, krule, float(eps),
             ptr(dxq), ptr(dxk), ptr(dxv), ptr(deta), ptr(dW), ptr(db), ptr(dlw), ptr(dlb),
-            ptr(saved), saved.numel(), stream_of(dev))
+            ptr(saved), saved.numel(), ptr(ws) if nws else None, nws, stream_of(dev))
     _lib.check(st, "ttt_linear_bwd")
     if sum_ln:
         dlw, dlb = dln.sum(1)

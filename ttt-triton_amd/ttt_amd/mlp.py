@@ -63,12 +63,11 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     saved or None).  ckpt, last and saved are what mlp_backward needs: the
     checkpoints every G mini-batches, the final state, and each mini-batch's
     state-update operands and activations (a flat uint8 buffer of
-    ttt_mlp_saved_bytes).  The backward reads only W1's checkpoints: with
+    ttt_mlp_saved_bytes, or of ttt_slots_bytes as _lib.slot_saved has it).  The backward reads only W1's checkpoints: with
     ckpt_w1_only the other three are neither allocated nor written (None).
     With `split` (fp32, K = 16; F = 64 with FF 64 or 256, F = 32 with FF = 128)
     the state and the readout run as two launches (TTT_FORM_SPLIT): the saved
-    buffer is then ttt_split_saved_bytes long, always allocated, and all that a
-    split backward needs."""
+    buffer is then always allocated, and all that a split backward needs."""
     rule = _lib.eta_rule_code(eta_rule)
     B, H, NC, K, F, FF = _check_shapes(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, rule)
     dev = check_device(XQ, XK, XV, eta, W1, b1, W2, b2, ln_w, ln_b)
@@ -97,10 +96,11 @@ def mlp_forward(ln_w, ln_b, W1, b1, W2, b2, XQ, XV, XK, eta, G: int, M: int = 0,
     saved = None
     if split:
         krule |= _lib.FORM_SPLIT
-    if want_saved or split or not _lib.fast_mlp_shape(K, F, FF):
-        nbytes = (lib.ttt_split_saved_bytes(B, H, NC, K, F, FF) if split
-                  else lib.ttt_mlp_saved_bytes(B, H, NC, K, F, FF, code))
-        saved = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    general = split or not _lib.fast_mlp_shape(K, F, FF)
+    if want_saved or general:
+        nbytes, form = _lib.slot_saved(B, H, NC, K, F, FF, split, train=want_saved) if general else (0, 0)
+        krule |= form
+        saved = torch.empty(nbytes or lib.ttt_mlp_saved_bytes(B, H, NC, K, F, FF, code), device=dev, dtype=torch.uint8)
     with on_device(dev):
         st = lib.ttt_mlp_fwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb), ptr(w1), ptr(bb1), ptr(w2), ptr(bb2),
@@ -119,7 +119,8 @@ def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, e
     """Run the backward kernel.  ckpt = (W1, b1, W2, b2) checkpoints, last =
     the final state and saved = the saved buffer, all from one mlp_forward
     call with the same G and eta form.  `workspace` (uint8, at least
-    ttt_mlp_bwd_workspace_bytes) is allocated here when not given; for the
+    ttt_mlp_bwd_workspace_bytes) is allocated here when not given, or where it
+    is too small for a `saved` of the slots alone; for the
     register-resident shapes (F = FF = 32) one of at least 256 bytes runs
     their one-launch backward instead of the two-launch one.  Returns
     fp32 (dln_w [H,F], dln_b [H,F], dW1, db1, dW2, db2) and (dXQ, dXV, dXK,
@@ -150,8 +151,12 @@ def mlp_backward(ln_w, ln_b, XQ, XV, XK, eta, ckpt, last, saved, dout, G: int, e
     dln = torch.empty((2, B, H, F), **f32)
     dlw, dlb = dln
     lib = _lib.load()
-    nws = 0 if split else lib.ttt_mlp_bwd_workspace_bytes(B, H, NC, K, F, FF, code)
-    ws = torch.empty(nws, device=dev, dtype=torch.uint8) if workspace is None else workspace
+    general = split or not _lib.fast_mlp_shape(K, F, FF)
+    nws, form = _lib.slot_workspace(saved, B, H, NC, K, F, FF, split) if general else (0, 0)
+    krule |= form
+    if workspace is None and not split:
+        nws = nws or lib.ttt_mlp_bwd_workspace_bytes(B, H, NC, K, F, FF, code)
+    ws = torch.empty(nws, device=dev, dtype=torch.uint8) if workspace is None or workspace.numel() < nws else workspace
     with on_device(dev):
         st = lib.ttt_mlp_bwd(
             ptr(xq), ptr(xk), ptr(xv), ptr(et), ptr(lw), ptr(lb),
