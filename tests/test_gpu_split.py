@@ -113,6 +113,40 @@ def test_rule():
     assert _lib.split_form(x(1, 1, nc, 16, 64), 0) and not _lib.split_form(x(1, 1, nc + 1, 16, 64), 0)
 
 
+def test_rule_of_short_sequences():
+    """From 3 mini-batches on; the MLP with at most 8 chains for each."""
+    from ttt_amd import _lib
+    x = lambda *s: torch.empty(s, dtype=F32, device="meta")  # noqa: E731
+    for F_, FF in ((64, 0), (64, 64), (64, 256), (32, 128)):
+        for NC in (1, 2):
+            assert not _lib.split_form(x(1, 1, NC, 16, F_), FF)
+        assert _lib.split_form(x(2, 4, 3, 16, F_), FF)
+    assert _lib.split_form(x(2, 64, 3, 16, 64), 0)
+    for F_, FF in ((64, 64), (32, 128)):
+        for NC in (3, 4, 7):
+            assert _lib.split_form(x(8, NC, NC, 16, F_), FF) and not _lib.split_form(x(1, 8 * NC + 1, NC, 16, F_), FF)
+    assert not _lib.split_form(x(1, 25, 3, 16, 64), 256) and _lib.split_form(x(1, 32, 4, 16, 64), 256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("F_,FF", [(64, 0), (64, 256)])
+def test_inference_allocates_the_slots_alone(F_, FF):
+    """No handoff, no gradient buffers: `saved` is what a forward alone needs."""
+    from ttt_amd import _lib
+    from ttt_amd.linear import linear_forward
+    from ttt_amd.mlp import mlp_forward
+    B, H, NC = 2, 3, 5
+    g = to_dev(_inputs(B, H, NC, 16, F_, FF, F32, "layer", 7))
+    res = []
+    for want in (False, True):
+        r = (mlp_forward(*(g[k] for k in MLP_KEYS), 2, want_saved=want, split=True) if FF else
+             linear_forward(*(g[k] for k in LIN_KEYS), 2, want_saved=want, split=True))
+        full, slots = _lib.slot_bytes(B, H, NC, 16, F_, FF, True)
+        assert r[-1].numel() == (full if want else slots)
+        res.append(r[0])
+    assert torch.equal(*res)
+
+
 def test_abi_refuses_what_the_split_form_does_not_take():
     from ttt_amd import _lib
     lib = _lib.load()

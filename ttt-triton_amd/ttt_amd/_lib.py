@@ -158,7 +158,7 @@ def slot_workspace(saved, *shape_split):
     return (full, SAVED_SLOTS) if slots and saved.numel() == slots else (0, 0)
 
 
-# The split form's `saved` buffer and handoff are bounded: they hold every mini-batch's state.
+# The split form's `saved` is bounded: it holds every mini-batch's state.
 SPLIT_MAX_BYTES = 1 << 30
 
 
@@ -166,17 +166,28 @@ def split_form(XQ, FF: int) -> bool:
     """Whether 16-token mini-batches in fp32 run the split form (FORM_SPLIT; FF = 0:
     the Linear loop).  One chain is one workgroup of the specialised kernels,
     whose readout shares that workgroup's time with the recurrence; the split
-    form runs it on the rest of the GPU, and loses once the chains fill that.
-    Kernel times specialised / split, 32 mini-batches, forward + backward at
-    8, 64, 128 (96) chains: Linear 342/195, 348/239, 353/338 us (192 chains:
-    359/415); MLP F = FF = 64 547/378, 559/474, (579/581); F = 32, FF = 128
-    734/479, 741/584, (758/705); F = 64, FF = 256 1241/946 at 8, 1253/1114 at 32,
-    1275/1342 at 64.  In 16 bits the specialised kernels' shorter products win at
-    every count (Linear 120/198 at 8 chains)."""
-    most = 32 if FF == 256 else 64 if FF else 128
-    if XQ.dim() != 5 or XQ.dtype != torch.float32 or XQ.shape[0] * XQ.shape[1] > most:
+    form runs it on the rest of the GPU, and loses once the chains fill that, or
+    where there is hardly a recurrence to run beside.  Specialised / split, us in a
+    captured graph, forward + backward at 8, 64, 128 (MLP, F = 64, FF = 256: 8, 32)
+    chains of 32 mini-batches, then the forward alone:
+      Linear       349/197, 356/242, 356/329    126/64, 128/79, 128/94
+      MLP 64/64    559/384, 568/462             185/139, 187/161
+      MLP 32/128   757/483, 765/571             279/155, 281/180
+      MLP 64/256   1,239/946, 1,249/1,118       434/304, 436/329
+    Short sequences, the forward alone:
+      Linear       1 mini-batch 12/19 (1 chain), 2: 16/19, 3: 20/18 (64 chains), 4: 23/20
+      MLP 64/64    2: 19/22 (8), 3: 25/25 (8) 25/29 (64), 4: 30/32 (32) 30/34 (64), 8: 53/55 (64), 12: 75/73 (64)
+      MLP 64/256   2: 36/40 (8), 3: 50/49 (8) 50/54 (32), 4: 63/64 (32), 6: 90/81 (32)
+    so it takes 3 mini-batches, and of the MLP no more than 8 chains for each.  The
+    rule is the same with and without a backward, and so are the outputs.  In 16
+    bits the specialised kernels' shorter products win at every count."""
+    if XQ.dim() != 5 or XQ.dtype != torch.float32:
         return False
-    return 0 < load().ttt_split_saved_bytes(*XQ.shape, FF) <= SPLIT_MAX_BYTES
+    chains, NC = XQ.shape[0] * XQ.shape[1], XQ.shape[2]
+    most = min(32 if FF == 256 else 64, 8 * NC) if FF else 128
+    if chains > most or NC < 3:
+        return False
+    return 0 < slot_bytes(*XQ.shape, FF, True)[0] <= SPLIT_MAX_BYTES
 
 
 def eta_rule_code(rule) -> int:
