@@ -2,6 +2,9 @@
 what a forward needs, the backward's handoff beside or behind it, and the size
 past which the general-shape kernels run."""
 
+import os
+import subprocess
+
 import pytest
 import torch
 
@@ -19,6 +22,18 @@ def _sizes(K, F_, FF):
     if FF:
         return 2 * F_ * FF + FF + F_, 2 * K * (FF + F_) + K, 2 * F_ * FF + FF + F_ + 2 * K * (FF + F_) + 2 * F_ + K
     return F_ * F_ + F_, 2 * K * F_ + K, F_ * F_ + F_ + 2 * K * F_ + 2 * F_ + K
+
+
+def test_layout(tmp_path):
+    """Which wave reads which token's eta (never past the mini-batch), the slot's
+    parts, alignment, LDS size: csrc/ttt_wide_layout.h enumerated on the host."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    csrc = os.path.join(os.path.dirname(here), "ttt-triton_amd", "csrc")
+    exe = str(tmp_path / "check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", csrc, os.path.join(here, "wide_layout_check.cpp"), "-o", exe],
+                   check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert (r.returncode, r.stdout) == (0, "16\n"), r.stdout
 
 
 @pytest.mark.parametrize("split,shape", [(0, s) for s in SHAPES] + [(1, s) for s in SPLIT])

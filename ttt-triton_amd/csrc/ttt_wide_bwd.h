@@ -220,7 +220,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
   const vf lw = ldv<V>(a.ln_w + (size_t)h * F + pcol), lb = ldv<V>(a.ln_b + (size_t)h * F + pcol);
   const WideTile<4> ts(w);
   const WideTile<C::FT> tf(w);
-  const bool has_f = C::ALLF || w < C::KT * C::FT;
+  const bool has_f = C::f_tile(w);
   float* const slot0 = a.saved + chain * NC * (size_t)Sl::FLOATS;
   const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
   f4 dw1[NSL][NT], dw2[MLP ? NSL : 1][NT];
@@ -265,8 +265,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
     const vf zh = ldv<V>(slot + Sl::ZH + po);
     const float sd = (slot + Sl::SIG)[(unsigned)prow];
     const unsigned es = wide_eta_last_raw<T, K>(a, m, ts.row());
-    // (waves without a K x F tile have rows past the mini-batch, and past eta's end at the last one)
-    const unsigned ef = C::FT == 4 ? es : has_f ? wide_eta_last_raw<T, K>(a, m, tf.row()) : 0u;
+    const unsigned ef = C::FT == 4 ? es : has_f ? wide_eta_last_raw<T, K>(a, m, C::f_token(w, lane)) : 0u;
     if (tid < 2 * F) hln += (slot + Sl::HLW)[(unsigned)tid];  // (HLB follows HLW)
     const vf xk = actf<T, V>(rxk), g2 = rg2;
     stv<V>(XKs + prow * LF + pcol, xk);

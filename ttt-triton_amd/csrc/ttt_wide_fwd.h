@@ -55,7 +55,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
   const vf lw = ldv<V>(a.ln_w + (size_t)h * F + pcol), lb = ldv<V>(a.ln_b + (size_t)h * F + pcol);
   const WideTile<4> ts(w);        // its K x 64 tile
   const WideTile<C::FT> tf(w);    // its K x F tile
-  const bool has_f = C::ALLF || w < C::KT * C::FT;
+  const bool has_f = C::f_tile(w);
   const int NK = (NC + a.G - 1) / a.G, NS = (NC + a.M - 1) / a.M;
   float* const slot0 = a.saved + chain * NC * a.slot_stride;
 
@@ -370,7 +370,7 @@ template <typename T, class C> struct WideReadout {
     C1 = sm + 6 * C::KSLOT;
     prow = threadIdx.x >> 4;
     pcol = (threadIdx.x & 15) * V;
-    has_f = C::ALLF || w < C::KT * C::FT;
+    has_f = C::f_tile(w);
     has_k = C::ALLK || w < C::KT * C::KT;
   }
   __device__ __forceinline__ void stage_w1(int sl) {
