@@ -114,18 +114,22 @@ def test_rule():
 
 
 def test_rule_of_short_sequences():
-    """From 3 mini-batches on; the MLP with at most 8 chains for each."""
+    """Without a backward from 3 mini-batches on, the 64-wide MLPs with at most 6
+    chains for each; with one, the MLP of 256 units from 3 on."""
     from ttt_amd import _lib
     x = lambda *s: torch.empty(s, dtype=F32, device="meta")  # noqa: E731
     for F_, FF in ((64, 0), (64, 64), (64, 256), (32, 128)):
         for NC in (1, 2):
-            assert not _lib.split_form(x(1, 1, NC, 16, F_), FF)
-        assert _lib.split_form(x(2, 4, 3, 16, F_), FF)
-    assert _lib.split_form(x(2, 64, 3, 16, 64), 0)
-    for F_, FF in ((64, 64), (32, 128)):
-        for NC in (3, 4, 7):
-            assert _lib.split_form(x(8, NC, NC, 16, F_), FF) and not _lib.split_form(x(1, 8 * NC + 1, NC, 16, F_), FF)
-    assert not _lib.split_form(x(1, 25, 3, 16, 64), 256) and _lib.split_form(x(1, 32, 4, 16, 64), 256)
+            assert not _lib.split_form(x(1, 1, NC, 16, F_), FF, train=False)
+            assert _lib.split_form(x(1, 1, NC, 16, F_), FF) == (FF != 256)
+        assert _lib.split_form(x(2, 4, 3, 16, F_), FF) and _lib.split_form(x(2, 4, 3, 16, F_), FF, train=False)
+    assert _lib.split_form(x(2, 64, 3, 16, 64), 0, train=False) and _lib.split_form(x(1, 64, 3, 16, 32), 128, train=False)
+    for FF, most in ((64, 64), (256, 32)):
+        for NC in (3, 4, 5, 16):
+            n = min(6 * NC, most)
+            assert _lib.split_form(x(1, n, NC, 16, 64), FF, train=False)
+            assert not _lib.split_form(x(1, n + 1, NC, 16, 64), FF, train=False)
+            assert _lib.split_form(x(1, most, NC, 16, 64), FF)
 
 
 @pytest.mark.gpu

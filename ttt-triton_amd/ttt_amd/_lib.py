@@ -162,7 +162,7 @@ def slot_workspace(saved, *shape_split):
 SPLIT_MAX_BYTES = 1 << 30
 
 
-def split_form(XQ, FF: int) -> bool:
+def split_form(XQ, FF: int, train: bool = True) -> bool:
     """Whether 16-token mini-batches in fp32 run the split form (FORM_SPLIT; FF = 0:
     the Linear loop).  One chain is one workgroup of the specialised kernels,
     whose readout shares that workgroup's time with the recurrence; the split
@@ -174,20 +174,28 @@ def split_form(XQ, FF: int) -> bool:
       MLP 64/64    559/384, 568/462             185/139, 187/161
       MLP 32/128   757/483, 765/571             279/155, 281/180
       MLP 64/256   1,239/946, 1,249/1,118       434/304, 436/329
-    Short sequences, the forward alone:
-      Linear       1 mini-batch 12/19 (1 chain), 2: 16/19, 3: 20/18 (64 chains), 4: 23/20
-      MLP 64/64    2: 19/22 (8), 3: 25/25 (8) 25/29 (64), 4: 30/32 (32) 30/34 (64), 8: 53/55 (64), 12: 75/73 (64)
+    Short sequences, forward + backward (chains):
+      1 mini-batch: Linear 36/26 (8), MLP 64/64 41/40 (64), 32/128 49/46 (64), 64/256 67/80 (1)
+      2, 3:         MLP 64/256 114/121, 155/149 (32)
+    and the forward alone:
+      Linear       1 mini-batch 12/19 (1), 2: 16/19 (1), 3: 20/18 (64), 4: 23/20 (64)
+      MLP 64/64    2: 19/22 (8), 3: 25/25 (8) 25/29 (64), 4: 30/32 (32) 30/34 (64), 6: 41/40 (32), 8: 53/55 (64)
       MLP 64/256   2: 36/40 (8), 3: 50/49 (8) 50/54 (32), 4: 63/64 (32), 6: 90/81 (32)
-    so it takes 3 mini-batches, and of the MLP no more than 8 chains for each.  The
-    rule is the same with and without a backward, and so are the outputs.  In 16
-    bits the specialised kernels' shorter products win at every count."""
+      MLP 32/128   2: 25/27 (64), 3: 33/32 (64)
+    so the forward alone takes 3 mini-batches, and of the 64-wide MLPs at most 6
+    chains for each; a forward with a backward behind it, of the MLP 64/256, takes 3.
+    In 16 bits the specialised kernels' shorter products win at every count."""
     if XQ.dim() != 5 or XQ.dtype != torch.float32:
         return False
-    chains, NC = XQ.shape[0] * XQ.shape[1], XQ.shape[2]
-    most = min(32 if FF == 256 else 64, 8 * NC) if FF else 128
-    if chains > most or NC < 3:
+    B, H, NC, K, F = XQ.shape
+    if NC < 3 and (FF == 256 or not train):
         return False
-    return 0 < slot_bytes(*XQ.shape, FF, True)[0] <= SPLIT_MAX_BYTES
+    most = 32 if FF == 256 else 64 if FF else 128
+    if not train and FF and F == 64:
+        most = min(most, 6 * NC)
+    if B * H > most:
+        return False
+    return 0 < slot_bytes(B, H, NC, K, F, FF, True)[0] <= SPLIT_MAX_BYTES
 
 
 def eta_rule_code(rule) -> int:

@@ -153,7 +153,7 @@ class TTTLinearFunction(torch.autograd.Function):
         G = min(max(int(checkpoint_group_size), 1), NC)
         # what the backward reads only when a gradient is wanted
         train = any(ctx.needs_input_grad)
-        split = _lib.split_form(XQ_batch, 0)
+        split = _lib.split_form(XQ_batch, 0, train)
         out, ck, last, saved = linear_forward(ttt_norm_weight, ttt_norm_bias, W1_init, b1_init, XQ_batch,
                                               XV_batch, XK_batch, eta_batch, G, eps, want_ckpt=train and not split,
                                               want_last=train and not split, want_saved=train, eta_rule=eta_rule,

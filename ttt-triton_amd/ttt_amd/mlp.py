@@ -198,7 +198,7 @@ class TTTMLPFunction(torch.autograd.Function):
         # what the backward reads (checkpoints, final state, saved buffer) only
         # when a gradient is wanted: an inference forward skips those stores
         train = any(ctx.needs_input_grad)
-        split = _lib.split_form(XQ_batch, W1_init.shape[-1])
+        split = _lib.split_form(XQ_batch, W1_init.shape[-1], train)
         keep = train and not split
         out, ck, memo, last, saved = mlp_forward(ttt_norm_weight, ttt_norm_bias, W1_init, b1_init, W2_init, b2_init,
                                                XQ_batch, XV_batch, XK_batch, eta_batch, G, M=M, eps=eps,
