@@ -314,21 +314,24 @@ def run_mlp(torch, steps, warmup, eta, only=None, Bn=B, memo=0, fwd_only=False, 
 
 
 def run_linear(torch, steps, warmup, eta, only=None, Bn=B, H_=H, NC_=NC, dtype=None, fwd_only=False):
+    from ttt_amd import _lib
     from ttt_amd.linear import linear_backward, linear_forward
     dev = torch.device("cuda:0")
     g = {k: v.to(dev) for k, v in make_inputs(torch, Bn, H_, NC_, F, seed=2, dtype=dtype, eta=eta).items()}
     keys = ("ln_w", "ln_b", "W1", "b1", "XQ", "XV", "XK", "eta")
     rule = "causal" if eta == "lr" else "dense"
+    split = _lib.split_form(g["XQ"], 0, train=not fwd_only)  # as TTTLinearFunction has it
+    keep = not fwd_only and not split
 
     def fwd():
-        out, ck, last, saved = linear_forward(*(g[k] for k in keys), min(G_LIN, NC_), want_ckpt=not fwd_only,
-                                              want_last=not fwd_only, want_saved=not fwd_only, eta_rule=rule)
+        out, ck, last, saved = linear_forward(*(g[k] for k in keys), min(G_LIN, NC_), want_ckpt=keep, want_last=keep,
+                                              want_saved=not fwd_only, eta_rule=rule, split=split)
         return out, (ck, last, saved)
 
     def bwd(st):
         ck, last, saved = st
-        return linear_backward(g["ln_w"], g["ln_b"], g["XQ"], g["XV"], g["XK"], g["eta"], ck[0], last[0], saved,
-                               g["dOut"], min(G_LIN, NC_), eta_rule=rule)
+        return linear_backward(g["ln_w"], g["ln_b"], g["XQ"], g["XV"], g["XK"], g["eta"], ck[0] if ck else None,
+                               last[0] if last else None, saved, g["dOut"], min(G_LIN, NC_), eta_rule=rule, split=split)
 
     _, ck = fwd()
     for _ in range(warmup):
@@ -378,7 +381,8 @@ def memo_pairs(M=MEMO_M):
 
 
 def run_memo(torch, steps, warmup, only=None):
-    from ttt_amd.memo import memo_combine_backward, memo_combine_forward
+    from ttt_amd.memo import (memo_combine_backward, memo_combine_backward_kept, memo_combine_forward, memo_rows,
+                              training_form)
     dev = torch.device("cuda:0")
     gen = torch.Generator().manual_seed(5)
     NS = math.ceil(NC / MEMO_M)
@@ -389,21 +393,35 @@ def run_memo(torch, steps, warmup, only=None):
           0.02 * torch.randn(B, H, NS, FF, F, generator=gen), torch.zeros(B, H, NS, 1, F)]
     ws = [w.to(dev) for w in ws]
     lw, lb = torch.ones(H, F, device=dev), torch.zeros(H, F, device=dev)
-    _, gates = memo_combine_forward(xq, xk, xu, xqw, *ws, lw, lb, MEMO_M)
+    n = memo_rows(B, H, NC, K, F, MEMO_M)
+    keep, images = training_form(n, FF, torch.bfloat16)
+
+    def fwd():  # as MemoCombineFunction calls them when gradients are wanted
+        rows = torch.empty(n, device=dev) if keep else None
+        _, gates = memo_combine_forward(xq, xk, xu, xqw, *ws, lw, lb, MEMO_M, images=images, rows=rows)
+        return gates, rows
+
+    def bwd(gates, rows):
+        if keep:
+            memo_combine_backward_kept(xq, xu, xqw, lw, lb, MEMO_M, gates, rows, dout)
+        else:
+            memo_combine_backward(xq, xu, xqw, *ws, lw, lb, MEMO_M, gates, dout)
+
+    st = fwd()
     for _ in range(warmup):
-        _, gates = memo_combine_forward(xq, xk, xu, xqw, *ws, lw, lb, MEMO_M)
-        memo_combine_backward(xq, xu, xqw, *ws, lw, lb, MEMO_M, gates, dout)
+        st = fwd()
+        bwd(*st)
     torch.cuda.synchronize()
     tm = Timer(torch)
     for _ in range(steps):
         if only != "memo_bwd":
             tm.mark("ttt_mlp_memo_combine")
-            _, gates = memo_combine_forward(xq, xk, xu, xqw, *ws, lw, lb, MEMO_M)
+            st = fwd()
         if only != "memo_fwd":
             tm.mark("ttt_mlp_memo_combine_bwd")
-            memo_combine_backward(xq, xu, xqw, *ws, lw, lb, MEMO_M, gates, dout)
+            bwd(*st)
         if only is None:
-            # the inference form: no backward follows, so no memo-state images
+            # the inference form: no backward follows, so neither rows nor images
             tm.mark("ttt_mlp_memo_combine_inference")
             memo_combine_forward(xq, xk, xu, xqw, *ws, lw, lb, MEMO_M, images=False)
     tm.mark(None)
