@@ -105,16 +105,14 @@ def test_which_forwards_take_the_slots_alone(monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dt", [F32, BF16])
-@pytest.mark.parametrize("split,K,F_,FF", [(0, *s) for s in SHAPES] + [(1, *s) for s in SPLIT])
+@pytest.mark.parametrize("split,K,F_,FF,dt", [(0, *s, dt) for s in SHAPES for dt in (F32, BF16)] +
+                         [(1, *s, F32) for s in SPLIT])
 def test_with_the_handoffs_place_and_without(monkeypatch, split, K, F_, FF, dt):
     """The same outputs and gradients, bitwise, from either `saved`, and
     of a second backward, which leaves the slots as they were."""
     from ttt_amd import _lib
     from ttt_amd.linear import linear_backward, linear_forward
     from ttt_amd.mlp import mlp_backward, mlp_forward
-    if split and dt != F32:
-        pytest.skip("the split form is fp32")
     B, H, NC, G = 2, 3, 5, 2
     g = to_dev(_inputs(B, H, NC, K, F_, FF, dt, "layer", K + FF))
     full, slots = _lib.slot_bytes(B, H, NC, K, F_, FF, bool(split))

@@ -83,11 +83,20 @@ __device__ __forceinline__ size_t pinned_index(size_t m) {
 // MFMA: left to itself the compiler waits for each pair of LDS reads in front of
 // its two MFMAs.  (With four waves per SIMD the others' MFMAs cover that, and the
 // batched reads queue: the MLP's state launches at K = F = FF = 64 took 10% more.)
+// The product is summed by itself and added to c once: added to c term by term, a
+// state took a rounding of its own size from each of the K terms of its update, and the
+// gradients of K = 64 were 2.2 to 2.6 times as far from 64 bits as the general-shape
+// kernels' (fp32, rms over five inputs: dXQ 2.6, dW1 2.2, out 2.2, now 1.0).  wmm_on
+// starts from c instead: a term of the sum's own size (zero, a bias); wmm_sl adds the
+// product of a hidden slice to the slices before it.  (The state launches of 16 tokens
+// go on with c throughout: four MFMAs a term, errors below the specialised kernels'
+// either way, and 8-10% less time.)
 // With CS, `cs` receives op(B)'s column sums (column r, in every lane group).
 // what may cross: VALU, SALU, VMEM, LDS writes; LDS reads and MFMAs may not
 constexpr int kSchedKeepLdsReads = 0x2 | 0x4 | 0x70 | 0x200;
-template <class C, int KD, bool TA, bool TB, int LA, int LB, bool CS = false>
+template <class C, int KD, bool TA, bool TB, int LA, int LB, bool CS = false, bool ON_ = false>
 __device__ __forceinline__ f4 wmm(f4 c, const float* A, const float* B, float* cs = nullptr) {
+  constexpr bool ON = ON_ || C::CHAIN;
   const int l = C::PIN ? pinned(lane_id()) : lane_id(), g = l >> 4, r = l & 15;
   const float* ap = TA ? A + 4 * g * LA + r : A + r * LA + 4 * g;
   const float* bp = TB ? B + r * LB + 4 * g : B + 4 * g * LB + r;
@@ -109,13 +118,31 @@ __device__ __forceinline__ f4 wmm(f4 c, const float* A, const float* B, float* c
   }
   if constexpr (C::KT == 1) __builtin_amdgcn_sched_barrier(kSchedKeepLdsReads);
   float t = 0.f;
+  f4 p = ON ? c : f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int k = 0; k < KD / 16; ++k) {
     if constexpr (CS) t += (b[k].v[0] + b[k].v[1]) + (b[k].v[2] + b[k].v[3]);
-    mma16(c, b[k], a[k]);
+    mma16(p, b[k], a[k]);
   }
   if constexpr (CS) *cs = sum_col4(t);
-  return c;
+  if constexpr (ON) {
+    return p;
+  } else {
+    // (c is taken up behind the product: brought forward it cost the FF = 256 backward 70
+    // spilled registers of 128 more)
+    asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]) : "v"(p[0]));
+    return c + p;
+  }
+}
+
+template <class C, int KD, bool TA, bool TB, int LA, int LB>
+__device__ __forceinline__ f4 wmm_on(f4 c, const float* A, const float* B) {
+  return wmm<C, KD, TA, TB, LA, LB, false, true>(c, A, B);
+}
+
+template <class C, int KD, bool TA, bool TB, int LA, int LB>
+__device__ __forceinline__ f4 wmm_sl(f4 c, const float* A, const float* B) {
+  return wmm<C, KD, TA, TB, LA, LB, false, (C::NSL == 1)>(c, A, B);
 }
 
 // this wave's index: uniform, below NW

@@ -67,12 +67,12 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
   f4 dxq = zero;              // of its K x F tile
   float* const DA = C::MLP ? ro.G2 : ro.W2;  // d(X2b X2^T), then d(XQ XK^T)
   if (C::ALLK || ro.has_k) {
-    const f4 dc = wmm<WideFree<C>, F, false, true, LF, LF>(zero, ro.Z + 16 * tk.it * LF, ro.G2 + 16 * tk.jt * LF);  // -dC
+    const f4 dc = wmm_on<WideFree<C>, F, false, true, LF, LF>(zero, ro.Z + 16 * tk.it * LF, ro.G2 + 16 * tk.jt * LF);  // -dC
     deta = -(dc * ((C::MLP ? ro.a2 : ro.a1) + 1.0f));
     da = -(dc * ro.eta);
   }
   if (C::ALLF || ro.has_f) {  // -C^T dZ2b
-    const f4 t = wmm<WideFree<C>, K, true, false, LK, LF>(zero, ro.C1 + 16 * tf.it, ro.Z + 16 * tf.jt);
+    const f4 t = wmm_on<WideFree<C>, K, true, false, LK, LF>(zero, ro.C1 + 16 * tf.it, ro.Z + 16 * tf.jt);
     stf4(tf.template at<F>(slot + Sl::HG2), t);
   }
   float cs;
@@ -91,10 +91,10 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       stf4(ts.template at<LS>(ro.X2), x2);
       stf4(ts.template at<LS>(ro.XB), ro.xb[sl]);
       __syncthreads();
-      f4 dz = wmm<WideFree<C>, F, false, true, LF, LF>(zero, ro.Z + 16 * ts.it * LF, ro.W2 + 16 * ts.jt * LF);
+      f4 dz = wmm_on<WideFree<C>, F, false, true, LF, LF>(zero, ro.Z + 16 * ts.it * LF, ro.W2 + 16 * ts.jt * LF);
       dz = wmm<WideFree<C>, K, false, false, LK, LS>(dz, DA + 16 * ts.it * LK, ro.X2 + 16 * ts.jt);
       dz *= ro.db[sl];
-      stf4(ts.template at<FF>(slot + Sl::HX2 + sl * 64), wmm<WideFree<C>, K, true, false, LK, LS>(zero, DA + 16 * ts.it, ro.XB + 16 * ts.jt));
+      stf4(ts.template at<FF>(slot + Sl::HX2 + sl * 64), wmm_on<WideFree<C>, K, true, false, LK, LS>(zero, DA + 16 * ts.it, ro.XB + 16 * ts.jt));
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
@@ -105,7 +105,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
             dw = wmm<WideFree<C>, K, true, false, LS, LF, true>(zero, ro.XB, ro.Z + 16 * t2.jt, &cs);
             if (lane < 16) slot[Sl::HST + Sl::B2 + 16 * t2.jt + lane] = cs;
           } else {
-            dw = wmm<WideFree<C>, K, true, false, LS, LF>(zero, ro.XB + 16 * t2.it, ro.Z + 16 * t2.jt);
+            dw = wmm_on<WideFree<C>, K, true, false, LS, LF>(zero, ro.XB + 16 * t2.it, ro.Z + 16 * t2.jt);
           }
           stf4(t2.template at<F>(slot + Sl::HST + Sl::W2 + sl * 64 * F), dw);
         }
@@ -115,9 +115,9 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       stf4(ts.template at<LS>(ro.X2), g1);
       ro.stage_w1(sl);
       __syncthreads();
-      if (C::ALLF || ro.has_f) dxq = wmm<WideFree<C>, C::S, false, true, LS, LS>(dxq, ro.XB + 16 * tf.it * LS, ro.W1 + 16 * tf.jt * LS);
-      if (C::ALLK || ro.has_k) dc1 = wmm<WideFree<C>, C::S, false, true, LS, LS>(dc1, ro.XB + 16 * tk.it * LS, ro.X2 + 16 * tk.jt * LS);
-      stf4(ts.template at<FF>(slot + Sl::HG1 + sl * 64), wmm<WideFree<C>, K, true, false, LK, LS>(zero, ro.C1 + 16 * ts.it, ro.XB + 16 * ts.jt));
+      if (C::ALLF || ro.has_f) dxq = wmm_sl<WideFree<C>, C::S, false, true, LS, LS>(dxq, ro.XB + 16 * tf.it * LS, ro.W1 + 16 * tf.jt * LS);
+      if (C::ALLK || ro.has_k) dc1 = wmm_sl<WideFree<C>, C::S, false, true, LS, LS>(dc1, ro.XB + 16 * tk.it * LS, ro.X2 + 16 * tk.jt * LS);
+      stf4(ts.template at<FF>(slot + Sl::HG1 + sl * 64), wmm_on<WideFree<C>, K, true, false, LK, LS>(zero, ro.C1 + 16 * ts.it, ro.XB + 16 * ts.jt));
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int t = w + n * C::NW;
@@ -128,7 +128,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
             dw = wmm<WideFree<C>, K, true, false, LF, LS, true>(zero, ro.XQ, ro.XB + 16 * t1.jt, &cs);
             if (lane < 16) slot[Sl::HST + Sl::B1 + sl * 64 + 16 * t1.jt + lane] = cs;
           } else {
-            dw = wmm<WideFree<C>, K, true, false, LF, LS>(zero, ro.XQ + 16 * t1.it, ro.XB + 16 * t1.jt);
+            dw = wmm_on<WideFree<C>, K, true, false, LF, LS>(zero, ro.XQ + 16 * t1.it, ro.XB + 16 * t1.jt);
           }
           stf4(t1.template at<FF>(slot + Sl::HST + Sl::W1 + sl * 64), dw);
         }
@@ -141,7 +141,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       stf4(tk.template at<LK>(DA), da);
     }
   } else {
-    dxq = wmm<WideFree<C>, F, false, true, LF, LS>(zero, ro.Z + 16 * tf.it * LF, ro.W1 + 16 * tf.jt * LS);
+    dxq = wmm_on<WideFree<C>, F, false, true, LF, LS>(zero, ro.Z + 16 * tf.it * LF, ro.W1 + 16 * tf.jt * LS);
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       const int t = w + n * C::NW;
@@ -152,7 +152,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
           dw = wmm<WideFree<C>, K, true, false, LF, LF, true>(zero, ro.XQ, ro.Z + 16 * t1.jt, &cs);
           if (lane < 16) slot[Sl::HST + Sl::B1 + 16 * t1.jt + lane] = cs;
         } else {
-          dw = wmm<WideFree<C>, K, true, false, LF, LF>(zero, ro.XQ + 16 * t1.it, ro.Z + 16 * t1.jt);
+          dw = wmm_on<WideFree<C>, K, true, false, LF, LF>(zero, ro.XQ + 16 * t1.it, ro.Z + 16 * t1.jt);
         }
         stf4(t1.template at<F>(slot + Sl::HST + Sl::W1), dw);
       }
@@ -182,7 +182,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
   if (C::ALLF || ro.has_f) {
     dxq = wmm<WideFree<C>, K, false, false, LK, LF>(dxq, DA + 16 * tf.it * LK, ro.XK + 16 * tf.jt);
     st4(tf.template at<F>(static_cast<T*>(a.dXQ) + m * K * F), dxq + frag_to_f4(ldraw4(tf.template at<F>(DO))));
-    stf4(tf.template at<F>(slot + Sl::HXK), wmm<WideFree<C>, K, true, false, LK, LF>(zero, DA + 16 * tf.it, ro.XQ + 16 * tf.jt));
+    stf4(tf.template at<F>(slot + Sl::HXK), wmm_on<WideFree<C>, K, true, false, LK, LF>(zero, DA + 16 * tf.it, ro.XQ + 16 * tf.jt));
   }
   if (lr_rule && tid < K) {
     float t = 0.f;
@@ -324,23 +324,23 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
         stage_w2(sl);
         __syncthreads();
         // through the update W1' = W1 - XK^T (e G1), b1' = b1 - G1^T e
-        const f4 t = wmm<C, F, false, false, LF, LS>(ldf4(db1s + sl * 64 + ts.col()), XKs + 16 * ts.it * LF,
+        const f4 t = wmm_on<C, F, false, false, LF, LS>(ldf4(db1s + sl * 64 + ts.col()), XKs + 16 * ts.it * LF,
                                                   DW1s + 16 * ts.jt);
         const f4 tg = t * g1;
         const float dpart = sum_col4((tg[0] + tg[1]) + (tg[2] + tg[3]));
         if (lane < 16) dep[ts.jt][ts.row()] = (sl == 0 ? 0.f : dep[ts.jt][ts.row()]) - dpart;
         const f4 dg1 = hg1 - t * e_s;
         dz1a[sl] = dg1 * p * dd1;
-        dx2[sl] = hx2 - wmm<C, F, false, true, LF, LF>(zero, G2s + 16 * ts.it * LF, DW2s + 16 * ts.jt * LF) * e_s;
+        dx2[sl] = hx2 - wmm_on<C, F, false, true, LF, LF>(zero, G2s + 16 * ts.it * LF, DW2s + 16 * ts.jt * LF) * e_s;
         if (has_f) {
-          t2 = wmm<C, C::S, false, false, LS, LF>(t2, X2s + 16 * tf.it * LS, DW2s + 16 * tf.jt);
-          dxk = wmm<C, C::S, false, true, LS, LS>(dxk, G1s + 16 * tf.it * LS, DW1s + 16 * tf.jt * LS);
+          t2 = wmm_sl<C, C::S, false, false, LS, LF>(t2, X2s + 16 * tf.it * LS, DW2s + 16 * tf.jt);
+          dxk = wmm_sl<C, C::S, false, true, LS, LS>(dxk, G1s + 16 * tf.it * LS, DW1s + 16 * tf.jt * LS);
         }
         __syncthreads();
         stf4(ts.template at<LS>(DW1s), dg1 * d1[sl]);  // dP
         if constexpr (NSL == 1) stage_w1(0);
         __syncthreads();
-        if (has_f) dg2 = wmm<C, C::S, false, false, LS, LF>(dg2, DW1s + 16 * tf.it * LS, W2s + 16 * tf.jt);
+        if (has_f) dg2 = wmm_sl<C, C::S, false, false, LS, LF>(dg2, DW1s + 16 * tf.it * LS, W2s + 16 * tf.jt);
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const int tt = w + n * C::NW;
@@ -362,8 +362,8 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
       }
       stage_w1(0);
       __syncthreads();
-      t2 = wmm<C, F, false, false, LF, LS>(t2, XKs + 16 * tf.it * LF, DW1s + 16 * tf.jt);
-      dxk = wmm<C, F, false, true, LF, LS>(dxk, G2s + 16 * tf.it * LF, DW1s + 16 * tf.jt * LS);
+      t2 = wmm_on<C, F, false, false, LF, LS>(t2, XKs + 16 * tf.it * LF, DW1s + 16 * tf.jt);
+      dxk = wmm_on<C, F, false, true, LF, LS>(dxk, G2s + 16 * tf.it * LF, DW1s + 16 * tf.jt * LS);
     }
     if (has_f) {
       t2 += ldf4((MLP ? db2s : db1s) + tf.col());

@@ -193,7 +193,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
           stage_w2(sl);
         }
         __syncthreads();
-        f4 z = wmm<C, F, false, false, LF, LS>(ldf4(b1s + sl * 64 + ts.col()), XKs + 16 * ts.it * LF, W1s + 16 * ts.jt);
+        f4 z = wmm_on<C, F, false, false, LF, LS>(ldf4(b1s + sl * 64 + ts.col()), XKs + 16 * ts.it * LF, W1s + 16 * ts.jt);
         stf4(ts.template at<FF>(slot + Sl::Z1 + sl * 64), z);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -205,11 +205,11 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
         stf4(ts.template at<LS>(X2s), x2[sl]);
         __syncthreads();
         if (has_f)
-          z2 = wmm<C, C::S, false, false, LS, LF>(z2, X2s + 16 * tf.it * LS, W2s + (sl & 1) * C::SLOT + 16 * tf.jt);
+          z2 = wmm_sl<C, C::S, false, false, LS, LF>(z2, X2s + 16 * tf.it * LS, W2s + (sl & 1) * C::SLOT + 16 * tf.jt);
       }
     } else {
       __syncthreads();
-      z2 = wmm<C, F, false, false, LF, LS>(z2, XKs + 16 * tf.it * LF, W1s + 16 * tf.jt);
+      z2 = wmm_on<C, F, false, false, LF, LS>(z2, XKs + 16 * tf.it * LF, W1s + 16 * tf.jt);
     }
     if (has_f) stf4(tf.template at<LF>(G2s), z2);
     // the next mini-batch's inputs are requested here and used after its barrier
@@ -277,7 +277,7 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_fw
           stf4(ts.template at<LS>(x2s), x2[sl]);
         }
         __syncthreads();
-        const f4 p = wmm<C, F, false, true, LF, LF>(f4{0.f, 0.f, 0.f, 0.f}, G2s + 16 * ts.it * LF, w2s + 16 * ts.jt * LF);
+        const f4 p = wmm_on<C, F, false, true, LF, LF>(f4{0.f, 0.f, 0.f, 0.f}, G2s + 16 * ts.it * LF, w2s + 16 * ts.jt * LF);
         stf4(ts.template at<FF>(slot + Sl::P + sl * 64), p);
         stf4(ts.template at<LS>(U1s), p * d1[sl] * -e_s);
         __syncthreads();
@@ -429,7 +429,7 @@ template <typename T, class C> struct WideReadout {
     __syncthreads();
     const f4 zero = f4{0.f, 0.f, 0.f, 0.f};
     if (C::ALLK || has_k) {
-      a1 = wmm<WideFree<C>, F, false, true, LF, LF>(zero, XQ + 16 * tk.it * LF, XK + 16 * tk.jt * LF);
+      a1 = wmm_on<WideFree<C>, F, false, true, LF, LF>(zero, XQ + 16 * tk.it * LF, XK + 16 * tk.jt * LF);
       stf4(tk.template at<LK>(C1), -(eta * (a1 + 1.0f)));
     }
     f4 z = zero;
@@ -438,7 +438,7 @@ template <typename T, class C> struct WideReadout {
 #pragma unroll
       for (int sl = 0; sl < NSL; ++sl) {
         f4 zb = ldf4(slot + Sl::B1 + sl * 64 + ts.col());
-        zb = wmm<WideFree<C>, F, false, false, LF, LS>(zb, XQ + 16 * ts.it * LF, W1 + 16 * ts.jt);
+        zb = wmm_on<WideFree<C>, F, false, false, LF, LS>(zb, XQ + 16 * ts.it * LF, W1 + 16 * ts.jt);
         if (sl == 0) __syncthreads();  // C1
         zb = wmm<WideFree<C>, K, false, false, LK, LS>(zb, C1 + 16 * ts.it * LK, Z + 16 * ts.jt);
 #pragma unroll
@@ -450,8 +450,8 @@ template <typename T, class C> struct WideReadout {
         }
         stf4(ts.template at<LS>(XB), xb[sl]);
         __syncthreads();
-        if (C::ALLK || has_k) a2 = wmm<WideFree<C>, C::S, false, true, LS, LS>(a2, XB + 16 * tk.it * LS, X2 + 16 * tk.jt * LS);
-        if (C::ALLF || has_f) z = wmm<WideFree<C>, C::S, false, false, LS, LF>(z, XB + 16 * tf.it * LS, W2 + 16 * tf.jt);
+        if (C::ALLK || has_k) a2 = wmm_sl<WideFree<C>, C::S, false, true, LS, LS>(a2, XB + 16 * tk.it * LS, X2 + 16 * tk.jt * LS);
+        if (C::ALLF || has_f) z = wmm_sl<WideFree<C>, C::S, false, false, LS, LF>(z, XB + 16 * tf.it * LS, W2 + 16 * tf.jt);
         if (sl + 1 < NSL) {
           __syncthreads();
           stage_w1(sl + 1);
@@ -467,7 +467,7 @@ template <typename T, class C> struct WideReadout {
         stf4(tf.template at<LF>(Z), z);
       }
     } else {
-      z = wmm<WideFree<C>, F, false, false, LF, LS>(z, XQ + 16 * tf.it * LF, W1 + 16 * tf.jt);
+      z = wmm_on<WideFree<C>, F, false, false, LF, LS>(z, XQ + 16 * tf.it * LF, W1 + 16 * tf.jt);
       __syncthreads();
       z = wmm<WideFree<C>, K, false, false, LK, LF>(z, C1 + 16 * tf.it * LK, G2 + 16 * tf.jt);
       stf4(tf.template at<LF>(Z), z);

@@ -21,6 +21,8 @@ template <int KT_, int FT_, int NSL_, bool MLP_> struct WideShape {
   // the state launches of 16 waves, MLP: addresses out of the registers (see pinned:
   // backward at K = F = FF = 64, B32 H4, 8 mini-batches 247 -> 172 us)
   static constexpr bool PIN = KT == 4 && MLP;
+  // the state launches' products onto a state: term by term (see wmm)
+  static constexpr bool CHAIN = KT == 1;
   // LDS rows are padded by 4 floats: row-major float4 reads (16 rows x 4 lane
   // groups) and column reads (4 rows x 16 lanes) both touch 64 distinct banks
   static constexpr int LS = S + 4, LF = F + 4, LK = K + 4;
@@ -36,8 +38,8 @@ template <int KT_, int FT_, int NSL_, bool MLP_> struct WideShape {
 
 // the readout launches, which have registers to spare and no loop: not pinned
 template <class C> struct WideFree {
-  static constexpr int KT = C::KT;
-  static constexpr bool PIN = false;
+  static constexpr int KT = C::KT, NSL = C::NSL;
+  static constexpr bool PIN = false, CHAIN = false;
 };
 
 // floats of one (chain, mini-batch) slot of `saved`: what the forward writes, then
