@@ -271,7 +271,7 @@ size_t wide_saved_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp);
 size_t wide_slots_bytes(int B, int H, int NC, int K, int F, int FF, bool mlp);
 hipError_t launch_wide_fwd(const GenFwdParams& p, int dtype, hipStream_t stream);
 hipError_t launch_wide_bwd(const GenBwdParams& p, int dtype, hipStream_t stream);
-bool gen_force_general();  // TTT_OPT_SMALL_KERNELS = 0: always the staged general-shape kernels
+bool gen_force_general();  // TTT_OPT_SMALL_KERNELS = 0: the register-resident kernels' shapes run the general ones
 hipError_t launch_small_fwd(const GenFwdParams& p, int dtype, hipStream_t stream);
 hipError_t launch_small_bwd(const GenBwdParams& p, int dtype, hipStream_t stream);
 

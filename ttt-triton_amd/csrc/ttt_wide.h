@@ -18,11 +18,18 @@
 // (the Linear loop has one layer: G, no P; the same four launches.)
 //
 // Measured at B32 H4, 8 mini-batches of 64 tokens, F = FF = 64, bf16, forward +
-// backward: 431 us (MLP; state 76 + 172, readouts 53 + 130), where the
+// backward: 429 us (MLP; state 77 + 172, readouts 53 + 132), where the
 // general-shape kernels (one workgroup per chain for everything, every matrix
 // through global scratch) take 6,780; the Linear loop 201 us against 3,090.
 // The shapes taken are those that a layer (FF = F) or the 4x MLP builds of
-// 32- and 64-wide heads; others keep the general-shape kernels.
+// 32- and 64-wide heads; others keep the general-shape kernels.  64 chains of 8
+// mini-batches, bf16, general-shape / these, us in a captured graph, forward and
+// forward + backward (1 and 192 chains, 1 and 2 mini-batches and fp32 alike; none
+// was slower here):
+//           Linear 64            MLP 64/64             MLP 64/256               MLP 32/128
+//   K = 32  385/38  1,379/99     815/67  2,906/190     2,838/191  10,199/922    889/77   3,176/228
+//   K = 48  549/49  2,017/128  1,122/85  4,380/296     4,069/351  14,465/1,468  1,307/100  5,100/391
+//   K = 64  719/55  2,685/149  1,478/99  5,934/314     5,530/361  19,796/1,597  1,805/118  6,915/446
 //
 // Mini-batches of 16 tokens in fp32 run here too where the caller asks for it
 // (the split form, TTT_FORM_SPLIT): one wave per SIMD, so every product's operands

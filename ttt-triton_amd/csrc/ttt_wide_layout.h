@@ -19,7 +19,8 @@ template <int KT_, int FT_, int NSL_, bool MLP_> struct WideShape {
   // whether every wave has a tile in each pass over them (no branch then)
   static constexpr bool ALLT = TW % NW == 0, ALLF = FT == 4, ALLK = KT == 4;
   // the state launches of 16 waves, MLP: addresses out of the registers (see pinned:
-  // backward at K = F = FF = 64, B32 H4, 8 mini-batches 247 -> 172 us)
+  // backward at K = F = FF = 64, B32 H4, 8 mini-batches 247 -> 172 us).  (K = 48 has 168
+  // registers a wave and spills 69 of the MLP's backward; not tried there.)
   static constexpr bool PIN = KT == 4 && MLP;
   // the state launches' products onto a state: term by term (see wmm)
   static constexpr bool CHAIN = KT == 1;

@@ -25,9 +25,10 @@ ttt_norm_weight/bias [H,F], post_norm, W1/b1/W2/b2), so a reference state
 dict loads unchanged.  Shapes the layer takes (ModelConfig raises ValueError
 for others): head dim F = model_dim / num_heads in {32, 64} (the producer,
 post-norm and memory-cache kernels), model_dim <= 1024, and a mini-batch
-size K that is a multiple of 16 up to 64.  The inner loop itself runs any
-shape on the general-shape kernels; K = 16 with F in {32, 64} (and the MLP's
-hidden width F, as TTTMLP builds it) runs on the specialised ones."""
+size K that is a multiple of 16 up to 64.  The layer's hidden width is F, as
+TTTMLP builds it: K = 16 runs on the specialised kernels (F = 32 MLP: the
+register-resident ones), K of 32 to 64 on the mini-batch-in-LDS kernels at F = 64
+and the register-resident ones at F = 32."""
 
 from __future__ import annotations
 
