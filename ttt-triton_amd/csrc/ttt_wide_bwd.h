@@ -201,7 +201,8 @@ template <typename T, class C> __global__ __launch_bounds__(C::NTH) void wide_bw
   typedef typename VecF<V>::type vf;
   typedef typename VecT<T, V>::type vt;
   __shared__ __align__(16) float sm[9 * C::SLOT];
-  __shared__ float db1s[FF], db2s[F], dep[8][K];
+  __shared__ __align__(16) float db1s[FF], db2s[F];
+  __shared__ float dep[8][K];
   float* const XKs = sm;
   float* const G2s = sm + C::SLOT;
   float* const DGs = sm + 2 * C::SLOT;   // dG2, then dZ2 in place
